@@ -220,3 +220,58 @@ def test_errors(gpu, tmp_path):
     path.write_bytes(bytes(img))
     with pytest.raises(ValueError, match="missing tensor model.layers.0.self_attn.q_proj.weight"):
         gpu.DecodeEngine(gpu.ModelFile(str(path)))
+
+
+# Where a step runs the split attention (from position 64 on): both sides of the switch, the first
+# and last position of a wave's tile of 64 and of a workgroup's 256, one and several heads per K/V
+# head, every head width, and a cache of more tiles than the grid has waves for.
+@pytest.mark.parametrize("shape,positions", [
+    (dict(n_heads=2, n_kv_heads=2, head_dim=64), 400),
+    (dict(n_heads=6, n_kv_heads=2, head_dim=64), 400),
+    (dict(n_heads=7, n_kv_heads=1, head_dim=128, qk_norm=True, biases=False), 400),
+    (dict(n_heads=2, n_kv_heads=1, head_dim=256, qk_norm=True), 330),
+    (dict(n_heads=2, n_kv_heads=1, head_dim=64), 33100),
+])
+def test_long_context_attention_matches_oracle(gpu, tmp_path, shape, positions):
+    """The split attention sums the positions in another order than attention_step (and the oracle),
+    in 32 bits with double sums of the probabilities, so the bar is the one of every step: 1e-4."""
+    from oracle.decode import DenseDecoder
+
+    class Decoder(DenseDecoder):
+        """One layer, whose k and v depend on the token alone: they are computed once per token, and a
+        step that is not checked only extends the cache."""
+        full, token, seen = False, 0, {}
+
+        def _mv(self, name, x, out_dim, in_dim):
+            if name.split(".")[-2] in ("q_proj", "k_proj", "v_proj"):
+                key = (name, self.token)
+                if key not in self.seen:
+                    self.seen[key] = super()._mv(name, x, out_dim, in_dim)
+                return self.seen[key].copy()
+            return super()._mv(name, x, out_dim, in_dim) if self.full else np.zeros(out_dim, np.float32)
+
+    def attend(q, *args):
+        from oracle.decode import attention_f64
+        return attention_f64(q, *args) if dec.full else np.zeros_like(q)
+
+    m, cfg, tensors = open_model(gpu, tmp_path, None, hidden=128, inter=256, vocab=100, layers=1,
+                                 max_seq_len=positions, **shape)
+    eng = gpu.DecodeEngine(m)
+    dec = Decoder(cfg, tensors, positions, exact_attention=False)
+    dec.seen, dec.attention = {}, attend
+    check = {63, 64, 65, 127, 128, 129, 255, 256, 257, 319, 320, 321, 32767, 32768, 32769, 33023, 33024, positions - 1}
+    tokens = [int(t) for t in np.random.default_rng(5).integers(0, 100, positions)]
+    first = {}
+    for i, t in enumerate(tokens):
+        tok = eng.step(t)
+        dec.full, dec.token = i in check, t
+        want = dec.step(t)
+        if i in check:
+            first[i] = eng.logits()
+            check_step(tok, first[i], want, (shape, i))
+    eng.reset()  # the same bits again, whichever part arrives last
+    for i, t in enumerate(tokens[:322]):
+        eng.step(t)
+        if i in first:
+            assert np.array_equal(eng.logits().view(np.uint32), first[i].view(np.uint32)), i
+    eng.close()
