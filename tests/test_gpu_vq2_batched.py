@@ -1,0 +1,56 @@
+"""The batched VQ2 product (matmul_vq2 of the "hip" variant, one launch for all tokens) against the
+oracle's matvec of every token.
+
+Bar: rel L2 <= 1e-5 and max|err| <= 1e-3 * max|y_ref|, as for the matvec: the same exact products
+with fp32 accumulation."""
+import numpy as np
+import pytest
+
+from conftest import max_abs_rel, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def product(orc, w, x, M, K, N):
+    return np.concatenate([orc.matvec_vq2(w, x[n * K:(n + 1) * K], M, K, threads=8) for n in range(N)])
+
+
+# rows and tokens around the 32-row and 32 / 64-token tiles; fewer chunks of 8 indices than waves, a
+# partial last chunk, index rows that are not dword-aligned (K % 16 != 0); one and two token blocks
+# per wave (9000 rows x 64 tokens: a workgroup per CU)
+@pytest.mark.parametrize("M,K,N", [(1, 4, 2), (31, 64, 2), (33, 36, 31), (100, 52, 33), (64, 1024, 65), (77, 1000, 5),
+                                   (896, 4864, 7), (9000, 272, 33), (9001, 260, 64), (4864, 896, 130)])
+def test_matches_oracle(gpu, orc, M, K, N):
+    w, x = gpu.synth_vq2(M, K, seed=M + K), gpu.synth_normal(K * N, seed=K + N)
+    got, want = gpu.matmul_vq2(w, x, M, K, N), product(orc, w, x, M, K, N)
+    assert rel_l2(got, want) <= 1e-5 and max_abs_rel(got, want) <= 1e-3
+    again = gpu.matmul_vq2(w, x, M, K, N)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+
+
+def test_token_blocks(gpu, orc):
+    """More tokens than one block of the workspaces holds (8M floats): the last block has one token."""
+    M, K = 260001, 8
+    N = (8 << 20) // M + 1
+    w, x = gpu.synth_vq2(M, K, seed=1), gpu.synth_normal(K * N, seed=2)
+    assert rel_l2(gpu.matmul_vq2(w, x, M, K, N), product(orc, w, x, M, K, N)) <= 1e-5
+
+
+@pytest.mark.parametrize("K", [896, 52])
+def test_non_finite_values_stay_where_they_are(gpu, orc, K):
+    """An infinite codebook entry 0 reaches exactly the rows that use it (positions past the row end
+    add nothing), a NaN activation exactly its token."""
+    M, N = 70, 35
+    w, x = gpu.synth_vq2(M, K, seed=3), gpu.synth_normal(K * N, seed=4)
+    w[0:8] = np.frombuffer(np.full(4, np.inf, np.float16).tobytes(), np.uint8)
+    x[3 * K + 1] = np.nan
+    got, want = gpu.matmul_vq2(w, x, M, K, N), product(orc, w, x, M, K, N)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin) and 0 < np.count_nonzero(fin) < want.size
+    assert rel_l2(got[fin], want[fin]) <= 1e-5
+
+
+def test_no_tokens_and_one_token(gpu):
+    w, x = gpu.synth_vq2(40, 64, seed=5), gpu.synth_normal(64, seed=6)
+    gpu.lib().tqhip_dispatch_matmul_vq2(w.ctypes.data, x.ctypes.data, None, 40, 64, 0)  # nothing to do
+    assert np.array_equal(gpu.matmul_vq2(w, x, 40, 64, 1), gpu.matvec_vq2(w, x, 40, 64))

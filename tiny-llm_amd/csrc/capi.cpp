@@ -12,6 +12,7 @@
 
 #include "../../include/tqhip.h"
 
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <mutex>
@@ -200,6 +201,35 @@ void download(HostBoundary &hb, const float *d, size_t n, const Piece *pieces, i
     }
     hb.read_split();
     for (int i = 0; i < np; ++i) std::memcpy(pieces[i].host, p + pieces[i].off, pieces[i].n * sizeof(float));
+}
+
+// matmul_vq2 of the "hip" variant: N > 1 tokens in blocks whose activations and outputs stay within
+// kBlockFloats each, so that the workspaces do not grow with the prompt.
+void matmul_vq2(const uint8_t *w, const float *x, float *y, int M, int K, int N) {
+    if (M < 1 || K < 4 || K % 4) check_status(kBadShape, "tqhip_matvec_vq2");
+    constexpr size_t kBlockFloats = size_t{8} << 20;
+    const int block = static_cast<int>(
+        std::min<size_t>(N, std::max<size_t>(1, kBlockFloats / static_cast<size_t>(std::max(M, K)))));
+    HostBoundary &hb = boundary();
+    std::lock_guard<std::mutex> lock(hb.mu);
+    hipStream_t s = hb.get_stream();
+    const uint8_t *dw = hb.resident(w, vq2_bytes(M, K));
+    for (int n0 = 0; n0 < N; n0 += block) {
+        const int n = std::min(block, N - n0);
+        const size_t nx = static_cast<size_t>(n) * K, ny = static_cast<size_t>(n) * M;
+        float *dx = hb.ensure(hb.dx, hb.x_cap, nx);
+        float *dy = hb.ensure(hb.dy, hb.y_cap, ny);
+        upload(hb, dx, x + static_cast<size_t>(n0) * K, nx, s);
+        int st = n > 1 ? launch_vq2_matmul(dw, dx, dy, M, K, n, s) : static_cast<int>(kNotFused);
+        if (st == kNotFused) {
+            st = kOk;
+            for (int i = 0; i < n && st == kOk; ++i)
+                st = launch_vq2_matvec(dw, dx + static_cast<size_t>(i) * K, dy + static_cast<size_t>(i) * M, M, K, s);
+        }
+        check_status(st, "tqhip_matmul_vq2");
+        const Piece out[1] = {{y + static_cast<size_t>(n0) * M, 0, ny}};
+        download(hb, dy, ny, out, 1, s);
+    }
 }
 
 }  // namespace
@@ -618,5 +648,6 @@ TINYQWEN_MATVEC_I4_VARIANT(tqhip_matvec_i4, "hip");
 TINYQWEN_MATVEC_I4_PAIR_VARIANT(tqhip_matvec_pair_i4, "hip");
 TINYQWEN_MATVEC_QKV_I4_VARIANT(tqhip_matvec_qkv_i4, "hip");
 TINYQWEN_MATVEC_VQ2_VARIANT(tqhip_matvec_vq2, "hip");
+TINYQWEN_MATMUL_VQ2_VARIANT(matmul_vq2, "hip");
 TINYQWEN_MATMUL_I4_VARIANT(tqhip_matmul_i4, "hip");
 TINYQWEN_BIIP_ROTATE_VARIANT(tqhip_biip_rotate, "hip");

@@ -73,6 +73,10 @@ Family<MatvecVQ2Fn> &vq2() {
     static Family<MatvecVQ2Fn> f;
     return f;
 }
+std::map<std::string, MatmulVQ2Fn> &mm_vq2() {
+    static std::map<std::string, MatmulVQ2Fn> m;
+    return m;
+}
 Family<MatmulI4Fn> &mm_i4() {
     static Family<MatmulI4Fn> f;
     return f;
@@ -134,7 +138,13 @@ void matvec_qkv_vq2(const uint8_t *wq, const uint8_t *wk, const uint8_t *wv, con
     matvec_vq2(wk, x, yk, kv_dim, in_dim);
     matvec_vq2(wv, x, yv, kv_dim, in_dim);
 }
+void register_matmul_vq2_impl(const char *name, MatmulVQ2Fn fn) { mm_vq2()[name] = fn; }
 void matmul_vq2(const uint8_t *w, const float *x, float *y, int M, int K, int N) {
+    auto it = mm_vq2().find(matvec_vq2_impl_name());
+    if (it != mm_vq2().end() && N > 1) {
+        it->second(w, x, y, M, K, N);
+        return;
+    }
     for (int n = 0; n < N; ++n)
         matvec_vq2(w, x + static_cast<size_t>(n) * K, y + static_cast<size_t>(n) * M, M, K);
 }

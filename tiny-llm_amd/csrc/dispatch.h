@@ -54,6 +54,10 @@ void matvec_pair_vq2(const uint8_t *w1, const uint8_t *w2, const float *x, float
                      int in_dim);
 void matvec_qkv_vq2(const uint8_t *wq, const uint8_t *wk, const uint8_t *wv, const float *x, float *yq, float *yk,
                     float *yv, int q_dim, int kv_dim, int in_dim);
+// A variant's batched product, used by matmul_vq2 when that variant is the selected matvec_vq2 (not in
+// the reference, whose matmul_vq2 is one matvec per token; a variant without one still is).
+using MatmulVQ2Fn = void (*)(const uint8_t *w, const float *x, float *y, int M, int K, int N);
+void register_matmul_vq2_impl(const char *name, MatmulVQ2Fn fn);
 void matmul_vq2(const uint8_t *w, const float *x, float *y, int M, int K, int N);
 
 void register_matmul_i4_impl(const char *name, MatmulI4Fn fn);
@@ -85,5 +89,7 @@ void biip_rotate_activation(const float *x, float *y, int dim, const float *scal
     [[maybe_unused]] static const bool tqwen_reg_qkv_i4_##fn = (tinyqwen::register_matvec_qkv_i4_impl(name, fn), true)
 #define TINYQWEN_MATVEC_VQ2_VARIANT(fn, name) \
     [[maybe_unused]] static const bool tqwen_reg_vq2_##fn = (tinyqwen::register_matvec_vq2_impl(name, fn), true)
+#define TINYQWEN_MATMUL_VQ2_VARIANT(fn, name) \
+    [[maybe_unused]] static const bool tqwen_reg_mm_vq2_##fn = (tinyqwen::register_matmul_vq2_impl(name, fn), true)
 #define TINYQWEN_MATMUL_I4_VARIANT(fn, name) \
     [[maybe_unused]] static const bool tqwen_reg_mm_i4_##fn = (tinyqwen::register_matmul_i4_impl(name, fn), true)
