@@ -1,0 +1,34 @@
+"""The prefill GEMM's preparation and tile kernels at the sizes where their dispatch changes.
+
+Bar of a product: rel L2 <= 2e-3 against the oracle (both operands rounded to fp16 once or, at
+G = 64, the weights twice); two kernels that form the same sums in the same order: the same bits."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def matmul_dev(gpu, w, x, M, K, N, G, x_offset=0):
+    """tqhip_matmul_i4_dev with X x_offset floats past a 16-byte boundary."""
+    xb = np.zeros(K * N + 4, np.float32)
+    xb[x_offset:x_offset + K * N] = x
+    dw, dx, dy = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(xb), gpu.DeviceBuffer(4 * M * N)
+    gpu.lib().tqhip_memset(dy.ptr, 0xFF, 4 * M * N)  # every output must be written
+    gpu.matmul_i4_dev(dw, dx.ptr + 4 * x_offset, dy, M, K, N, G)
+    gpu.synchronize()
+    return dy.download(np.float32, M * N)
+
+
+# one, two, four and eight 8-element chunks a thread, at and past each limit; past 16384 elements
+# and with X off a 16-byte boundary one float at a time
+@pytest.mark.parametrize("K", [2048, 2052, 4096, 4100, 8192, 8196, 9728, 16384, 16388])
+@pytest.mark.parametrize("G", [64, 128])
+def test_x_conversion_by_row_length(gpu, orc, K, G):
+    M, N = 33, 35
+    w, x = gpu.synth_i4(M, K, G, seed=K), gpu.synth_normal(K * N, seed=K + 1)
+    x[K:2 * K] *= 1e-20
+    got = matmul_dev(gpu, w, x, M, K, N, G)
+    assert np.array_equal(got.view(np.uint32), matmul_dev(gpu, w, x, M, K, N, G, x_offset=1).view(np.uint32))
+    assert rel_l2(got, orc.matmul_i4(w, x, M, K, N, G, threads=8)) <= 2e-3

@@ -98,19 +98,21 @@ __global__ __launch_bounds__(256) void x_to_f16(const float *__restrict__ x, int
     if (threadIdx.x == 0) xinv[n] = ldexpf(1.f, -e);
 }
 
-// x_to_f16 for K % 4 == 0 and x 16-byte aligned: thread t takes 8-element chunks t and t + 256
-// (two 16-byte loads each) and stores each chunk's 8 fp16 values, in the chunk's slot order,
-// with one 16-byte store. The same exponent and the same per-element rounding as x_to_f16.
-template <bool PERM>
+// x_to_f16 for K % 4 == 0 and x 16-byte aligned: thread t takes 8-element chunks t + 256 i, i < CH
+// (two 16-byte loads each, all in flight together) and stores each chunk's 8 fp16 values, in the
+// chunk's slot order, with one 16-byte store. The same exponent and the same per-element rounding
+// as x_to_f16. Bound by memory: rows of 9728 at 3001 tokens (175 MB) 32 us, where two scalar passes
+// (x_to_f16_long, still used for rows past 16384 and unaligned ones) take 77.
+constexpr int kXVecMax = 8;  // chunks per thread: rows of up to 2048 kXVecMax elements
+template <bool PERM, int CH>
 __global__ __launch_bounds__(256) void x_to_f16_vec(const float *__restrict__ x, int K, int Kp,
                                                       _Float16 *__restrict__ xh, float *__restrict__ xinv) {
-    constexpr int kChunks = kXRegs / 8;  // 8-element chunks per thread (Kp <= 256 * kXRegs)
     const int n = blockIdx.x;
     const float4 *xc = reinterpret_cast<const float4 *>(x + static_cast<size_t>(n) * K);
-    float v[kChunks][8];
+    float v[CH][8];
     float m = 0.f;
 #pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
+    for (int i = 0; i < CH; ++i) {
         const int c = threadIdx.x + 256 * i;  // elements 8c .. 8c + 7
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(256) void x_to_f16_vec(const float *__restrict__ x,
     }
     uint4 *hc = reinterpret_cast<uint4 *>(xh + static_cast<size_t>(n) * Kp);
 #pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
+    for (int i = 0; i < CH; ++i) {
         const int c = threadIdx.x + 256 * i;
         if (8 * c >= Kp) continue;
         unsigned short o[8];
@@ -1191,6 +1193,25 @@ int matmul_by_columns(const uint8_t *w, const float *x, float *y, int M, int K, 
     return kOk;
 }
 
+// X's fp16 copy and per-token scales; perm: in the packed dequantization's k-slot order.
+template <bool PERM>
+void launch_x_to_f16(const float *x, int K, int Kp, int N, _Float16 *xh, float *xinv, hipStream_t stream) {
+    const bool vec = K % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;  // 16-byte loads
+    const auto kernel = vec && Kp <= 2048   ? x_to_f16_vec<PERM, 1>
+                        : vec && Kp <= 4096 ? x_to_f16_vec<PERM, 2>
+                        : vec && Kp <= 8192 ? x_to_f16_vec<PERM, 4>
+                        : vec && Kp <= 2048 * kXVecMax ? x_to_f16_vec<PERM, kXVecMax>
+                        : Kp <= 256 * kXRegs           ? x_to_f16<PERM>
+                                                       : x_to_f16_long<PERM>;
+    hipLaunchKernelGGL(kernel, dim3(N), dim3(256), 0, stream, x, K, Kp, xh, xinv);
+}
+void launch_x_to_f16(bool perm, const float *x, int K, int Kp, int N, _Float16 *xh, float *xinv, hipStream_t stream) {
+    if (perm)
+        launch_x_to_f16<true>(x, K, Kp, N, xh, xinv, stream);
+    else
+        launch_x_to_f16<false>(x, K, Kp, N, xh, xinv, stream);
+}
+
 // The MFMA path with X's fp16 copy and per-token scales at ws (prefill_scratch_bytes(K, N) bytes).
 int matmul_mfma(const uint8_t *w, const float *x, float *y, int M, int K, int N, int group_size, unsigned char *ws,
                 hipStream_t stream) {
@@ -1206,14 +1227,7 @@ int matmul_mfma(const uint8_t *w, const float *x, float *y, int M, int K, int N,
     // with 32-bit offsets.
     const int g64_bm = wn == 1 ? 32 : wn == 2 ? 128 : 256;
     const bool g64 = group_size == 64 && static_cast<size_t>(g64_bm) * rb + Kp * 2 * 32 * wn < (1ull << 31);
-    const bool lng = Kp > static_cast<size_t>(256 * kXRegs);
-    const bool vec = !lng && K % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;  // 16-byte loads
-    if (g64)
-        hipLaunchKernelGGL(lng ? x_to_f16_long<true> : vec ? x_to_f16_vec<true> : x_to_f16<true>, dim3(N), dim3(256), 0,
-                           stream, x, K, ikp, xh, xinv);
-    else
-        hipLaunchKernelGGL(lng ? x_to_f16_long<false> : vec ? x_to_f16_vec<false> : x_to_f16<false>, dim3(N), dim3(256),
-                           0, stream, x, K, ikp, xh, xinv);
+    launch_x_to_f16(g64, x, K, ikp, N, xh, xinv, stream);
     if (hipGetLastError() != hipSuccess) return kLaunchFailed;
     int st;
     if (g64) {
