@@ -5,7 +5,7 @@ G = 64, the weights twice); two kernels that form the same sums in the same orde
 import numpy as np
 import pytest
 
-from conftest import rel_l2
+from conftest import fp16_operand_bound_ok, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +32,19 @@ def test_x_conversion_by_row_length(gpu, orc, K, G):
     got = matmul_dev(gpu, w, x, M, K, N, G)
     assert np.array_equal(got.view(np.uint32), matmul_dev(gpu, w, x, M, K, N, G, x_offset=1).view(np.uint32))
     assert rel_l2(got, orc.matmul_i4(w, x, M, K, N, G, threads=8)) <= 2e-3
+
+
+# group sizes other than 64 on the tile kernel: rows and tokens around its three tiles (32 x 32,
+# 128 x 64, 256 x 96), a last group that K does not fill, one that leaves the second half of the
+# last step without a group (G = 32, K = 1056), groups across step boundaries (G = 96), fewer steps
+# than the ring holds
+@pytest.mark.parametrize("G", [32, 96, 128, 256])
+@pytest.mark.parametrize("M,K,N", [(1, 32, 1), (33, 64, 32), (31, 1056, 33), (129, 100, 128), (257, 1000, 129),
+                                   (300, 2560, 200), (4, 4864, 97)])
+def test_other_group_sizes(gpu, orc, M, K, N, G):
+    w, x = gpu.synth_i4(M, K, G, seed=M + K + G), gpu.synth_normal(K * N, seed=N)
+    got, want = matmul_dev(gpu, w, x, M, K, N, G), orc.matmul_i4(w, x, M, K, N, G, threads=8)
+    if M * N < 16:  # a handful of outputs: each within the fp16 operands' rounding of its products
+        assert fp16_operand_bound_ok(got, want, orc, w, x, M, K, N, G)
+    else:
+        assert rel_l2(got, want) <= 2e-3

@@ -10,17 +10,15 @@
 //      zero-padded to a multiple of 64 along K. The scale keeps fp16 clear of
 //      overflow and gives every token the full 11-bit significand; 2^-e_n is
 //      applied exactly in the epilogue.
-//   2. i4_matmul_mfma: workgroup tiles of BM weight rows x BN tokens, 64 K
-//      elements per step. Global -> LDS DMA brings each step's raw W slice
-//      (group headers + packed codes) and fp16 X slice into a ring of 2-4
-//      stages, issued stages - 1 steps ahead. Each wave dequantizes its W
-//      operands from the raw codes in LDS straight into registers as
-//      q * scale - zero * scale with one rounding to fp16 (v_fma_mix), and
-//      contracts with v_mfma_f32_32x32x16_f16 (fp32 accumulation).
+//   2. i4_matmul_direct: workgroup tiles of 32 weight rows a wave x BN tokens, 64 K elements per
+//      step. Each lane loads its row's codes and group header straight into registers, the fp16 X
+//      slice comes by DMA into an LDS ring, both some steps ahead; the A operands are
+//      dequantized in registers and contracted with v_mfma_f32_32x32x16_f16 (fp32
+//      accumulation).
 //      fp16 and bf16 MFMA run at the same rate on gfx950; fp16 keeps 8x
 //      finer rounding of both operands.
 // Up to 32 tokens at G = 64 (16-byte aligned X, K % 4 == 0): one launch that converts X
-// itself and splits K over workgroups (section 5 below).
+// itself and splits K over workgroups (section 3 below).
 // Other group sizes: one i4 matvec per token column.
 
 #include "i4_lane.h"
@@ -38,7 +36,6 @@ typedef float f16x __attribute__((ext_vector_type(16)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 
 constexpr int kStepK = 64;             // K elements per main-loop step
-constexpr int kThreads = 256;
 
 __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void *base, size_t bytes) {
     const int nrec = bytes > 0xFFFFFFFFull ? -1 : static_cast<int>(static_cast<unsigned>(bytes));
@@ -210,7 +207,7 @@ __device__ inline h8 dequant8(unsigned c, float s, float nzs) {
     return __builtin_bit_cast(h8, pk);
 }
 
-// ---- packed-fp16 dequantization (the G = 64 GEMM)
+// ---- packed-fp16 dequantization (G = 64)
 // A nibble q OR-ed into the mantissa of a fixed fp16 exponent reads as 1024 + q (bits 0..3 under
 // exponent 2^10) or 64 + q (bits 4..7 under 2^6), both exact; subtracting 1024 or 64 gives q
 // exactly, and fma(q, s, fp16(-z s)) rounds once. Eight elements cost 13 instructions (one shift,
@@ -292,365 +289,41 @@ __device__ inline void lds_barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-constexpr int kWDwords = 10;                    // per row and step
-constexpr int kWStage1 = 128 * kWDwords * 4;    // bytes of W per step and 128 rows
-constexpr int kWDma1 = 128 * kWDwords / 64 / 4; // dword DMAs per wave per step and 128 rows (= 5)
-
-// Byte offsets, within a row, of one step's W data: per 32-element half t the
-// group header and the first of its 16 code bytes (each half lies in one group
-// as G % 32 == 0). Uniform across the workgroup (scalar arithmetic).
-struct StepOffsets {
+// Byte offsets within a row of one step's two 32-element halves (each in one group, G % 32 == 0):
+// group header and 16 code bytes (scalar). Past the last group: the last one's, in the row (X is
+// zero there).
+struct HalfOffsets {
     int hdr[2], code[2];
-    bool valid[2];
 };
-template <int GT>
-__device__ __forceinline__ StepOffsets step_offsets(int s, int Grt, int gb, int groups) {
-    const int G = GT ? GT : Grt;  // a compile-time group size turns the divisions into shifts
-    StepOffsets o;
+__device__ __forceinline__ HalfOffsets half_offsets(int s, int G, int gb, int groups) {
+    HalfOffsets o;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int k = s * kStepK + 32 * t;
-        const int g = k / G;
-        o.valid[t] = g < groups;
-        const int gc = min(g, groups - 1);  // past the last group: any valid bytes, masked later
-        o.hdr[t] = gc * gb;
-        o.code[t] = gc * gb + 4 + (k - gc * G) / 2;
+        const int k = s * kStepK + 32 * t, g = min(k / G, groups - 1);
+        o.hdr[t] = g * gb;
+        o.code[t] = g * gb + 4 + min((k - g * G) / 2, G / 2 - 16);
     }
     return o;
 }
 
-// One step's global -> LDS DMAs of one wave (nw dword DMAs of W, nx 16-byte
-// DMAs of X, the X part starting xbase bytes into the stage); every lane of
-// every DMA is live, so the count per wave and step is fixed. Per lane only a
-// select and an add depend on the step. (Not a lambda in the kernel: HIP
-// compiles those for the host too, where the DMA builtin does not exist.)
-__device__ __forceinline__ void issue_step(__amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t xr, unsigned char *st,
-                                           const int *wrow, const int *wsel, int nw, const int *xoff, int nx,
-                                           int xbase, int wave, int s, const StepOffsets &o) {
-#pragma unroll
-    for (int q = 0; q < nw; ++q) {
-        // wsel: slot 0/1 -> header of half 0/1; slot 2+4t+i -> code dword i of half t
-        const int sl = wsel[q];
-        const int t = sl < 2 ? sl : (sl - 2) >> 2;
-        const int base = sl < 2 ? (t ? o.hdr[1] : o.hdr[0]) : (t ? o.code[1] : o.code[0]) + 4 * ((sl - 2) & 3);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            wr, (__attribute__((address_space(3))) void *)(st + 256 * (wave * nw + q)), 4, wrow[q] + base, 0, 0, 0);
-    }
-#pragma unroll
-    for (int q = 0; q < nx; ++q)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            xr, (__attribute__((address_space(3))) void *)(st + xbase + 1024 * (wave * nx + q)), 16,
-            xoff[q] + s * kStepK * 2, 0, 0, 0);
-}
-
-// ---- 2. MFMA tile kernel
-//   4 waves; wave w owns weight rows 32*WM*w .. +32*WM of the workgroup's
-//   BM = 128 * WM and all BN = 32 * WN tokens. Per 64-element K step,
-//   global -> LDS DMA brings
-//     W: per row 10 dwords [header of half 0, header of half 1, 8 code dwords]
-//        (each 32-element half lies in one group as G % 32 == 0);
-//     X: BN rows x 128 B of fp16, 16-byte chunks XOR-swizzled by row (c ^ (r & 7))
-//   into a ring of S stages issued S - 1 steps ahead. Each wave dequantizes its
-//   A operands from the raw codes in LDS straight into registers; every X (B)
-//   operand read from LDS feeds WM MFMAs.
-template <int WM, int WN, int GT>
-__global__ __launch_bounds__(kThreads) void i4_matmul_mfma(const uint8_t *__restrict__ w,
-                                                           const _Float16 *__restrict__ xh,
-                                                           const float *__restrict__ xinv, float *__restrict__ y,
-                                                           int M, int N, int K, int Kp, int G, int row_bytes, int S) {
-    constexpr int BM = 128 * WM;
-    constexpr int BN = 32 * WN;
-    constexpr int WStage = kWStage1 * WM;
-    constexpr int WDma = kWDma1 * WM;
-    constexpr int XStage = BN * 128;
-    constexpr int P = WDma + WN;  // DMAs per wave per step
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-    if constexpr (GT != 0) G = GT;
-    const int gb = 4 + G / 2;
-    const int groups = (K + G - 1) / G;
-    const int steps = Kp / kStepK;
-    const int stage_bytes = WStage + XStage;
-
-    const __amdgpu_buffer_rsrc_t wr = make_rsrc(w + static_cast<size_t>(m0) * row_bytes,
-                                                static_cast<size_t>(M - m0) * row_bytes);
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(xh + static_cast<size_t>(n0) * Kp,
-                                                static_cast<size_t>(N - n0) * Kp * 2);
-
-    // this wave's W DMAs: dword d = 64 * (wave * WDma + q) + lane of the stage
-    int wrow[WDma], wslot[WDma];
-#pragma unroll
-    for (int q = 0; q < WDma; ++q) {
-        const int d = 64 * (wave * WDma + q) + lane;
-        wrow[q] = (d / kWDwords) * row_bytes;
-        wslot[q] = d % kWDwords;
-    }
-    // this wave's X DMAs: 16-byte position p = 64 * (wave * WN + q) + lane
-    int xoff[WN];
-#pragma unroll
-    for (int q = 0; q < WN; ++q) {
-        const int p = 64 * (wave * WN + q) + lane;
-        const int r = p >> 3, c = (p & 7) ^ (r & 7);
-        xoff[q] = r * Kp * 2 + 16 * c;
-    }
-    auto issue = [&](int s, int slot) {
-        issue_step(wr, xr, smem + slot * stage_bytes, wrow, wslot, WDma, xoff, WN, WStage, wave, s,
-                   step_offsets<GT>(s, G, gb, groups));
-    };
-
-    f16x acc[WM][WN];
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = f16x{};
-
-    const int li = lane & 31, kq = lane >> 5;
-    int issued = 0;
-    for (; issued < S - 1 && issued < steps; ++issued) issue(issued, issued);
-    int slot = 0, islot = issued == S ? 0 : issued;  // ring slots of step s and of the next issue
-    for (int s = 0; s < steps; ++s) {
-        wait_vm((issued - s - 1) * P);  // this wave's part of step s has landed
-        lds_barrier();                  // every wave's part has; step s - 1's slot is free
-        if (issued < steps) {
-            issue(issued, islot);
-            ++issued;
-            islot = islot == S - 1 ? 0 : islot + 1;
-        }
-        const unsigned char *st = smem + slot * stage_bytes;
-        const StepOffsets so = step_offsets<GT>(s, G, gb, groups);
-        // all of the step's LDS operands first, so their latencies overlap
-        unsigned hd[WM][2], c[WM][4];
-#pragma unroll
-        for (int i = 0; i < WM; ++i) {
-            const unsigned *wrw = reinterpret_cast<const unsigned *>(st) + (32 * (WM * wave + i) + li) * kWDwords;
-            hd[i][0] = wrw[0];
-            hd[i][1] = wrw[1];
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) c[i][kk] = wrw[2 + 2 * kk + kq];
-        }
-        const unsigned char *sx = st + WStage;
-        h8 b[4][WN];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                const int r = 32 * j + li;
-                b[kk][j] = *reinterpret_cast<const h8 *>(sx + r * 128 + 16 * ((2 * kk + kq) ^ (r & 7)));
-            }
-#pragma unroll
-        for (int i = 0; i < WM; ++i) {
-            const float s0 = so.valid[0] ? half_bits_f(hd[i][0]) : 0.f;
-            const float s1 = so.valid[1] ? half_bits_f(hd[i][1]) : 0.f;
-            const float z0 = so.valid[0] ? -(half_bits_f(hd[i][0] >> 16) * s0) : 0.f;
-            const float z1 = so.valid[1] ? -(half_bits_f(hd[i][1] >> 16) * s1) : 0.f;
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                const h8 a = kk < 2 ? dequant8(c[i][kk], s0, z0) : dequant8(c[i][kk], s1, z1);
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[kk][j], acc[i][j], 0, 0, 0);
-            }
-        }
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    wait_vm(0);
-
-    // epilogue: lane holds rows (r/4)*8 + (lane/32)*4 + r%4 of column lane%32
-#pragma unroll
-    for (int j = 0; j < WN; ++j) {
-        const int n = n0 + 32 * j + li;
-        if (n >= N) continue;
-        const float sc = xinv[n];
-        float *yc = y + static_cast<size_t>(n) * M;
-#pragma unroll
-        for (int i = 0; i < WM; ++i)
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                const int m = m0 + 32 * (WM * wave + i) + 8 * r4 + 4 * kq;
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (m + q < M) yc[m + q] = acc[i][j][4 * r4 + q] * sc;
-            }
-    }
-}
-
-// ---- 3. MFMA tile kernel, slot-major staging
-//   The same tile, dequantization and MFMA as i4_matmul_mfma, with the per-step
-//   overhead taken out of the loop:
-//   - W is staged slot-major, [10 slots][128 rows] dwords (slot 0/1: group
-//     header of half 0/1 of the step; slot 2 + 4t + i: code dword i of half t).
-//     One DMA instruction moves one slot of 64 rows: its per-lane source is
-//     row * row_bytes, fixed for the whole loop, and the step enters only
-//     through the scalar offset of the slot (SALU), so no per-lane selects.
-//     Reading a slot back, 32 consecutive lanes read 32 consecutive dwords.
-//   - X rows are 128 B; 16-byte chunk c of token row r is stored at position
-//     c ^ ((r >> 1) & 7). A ds_read_b128 is served 16 lanes at a time, one
-//     256-byte bank sweep: the 16 rows a group reads differ in (r & 1, chunk),
-//     so they cover the sweep once (no bank conflicts).
-//   - Every step issues the same DMAs, also past the last step (reads past a
-//     row or the end of the buffer land in a slot that is never consumed), so
-//     the wait before each step is one constant s_waitcnt.
-constexpr int kWSlots = 10;
-constexpr int kBM = 128;
-
-// Byte offset within a row of the step-s dword of W slot `slot` (scalar).
-template <int GT>
-__device__ __forceinline__ int w_slot_offset(int slot, int s, int G, int gb, int groups) {
-    const int t = slot < 2 ? slot : (slot - 2) >> 2;
-    const int k = s * kStepK + 32 * t;
-    const int g = min(k / (GT ? GT : G), groups - 1);  // past the last group: in-row bytes, masked later
-    const int base = g * gb;
-    return slot < 2 ? base : base + 4 + (k - g * (GT ? GT : G)) / 2 + 4 * ((slot - 2) & 3);
-}
-
-// One step's DMAs of one wave: 5 W slot DMAs (instruction i = 5 * wave + q:
-// slot i >> 1, rows 64 (i & 1) + lane) and nx X DMAs of 16 bytes per lane.
-// (Not a template and not a lambda: the DMA builtin exists for the device only.)
-__device__ __forceinline__ void issue_step2(__amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t xr, unsigned char *st,
-                                            const int *wvo, const int *wso, const int *xvo, int nx, int xso,
-                                            int wstage, int wave) {
-#pragma unroll
-    for (int q = 0; q < 5; ++q)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            wr, (__attribute__((address_space(3))) void *)(st + 256 * (5 * wave + q)), 4, wvo[q], wso[q], 0, 0);
-#pragma unroll
-    for (int q = 0; q < nx; ++q)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            xr, (__attribute__((address_space(3))) void *)(st + wstage + 1024 * (nx * wave + q)), 16, xvo[q], xso, 0,
-            0);
-}
-
-template <int WN, int GT, int S>
-__global__ __launch_bounds__(kThreads) void i4_matmul_mfma2(const uint8_t *__restrict__ w,
-                                                            const _Float16 *__restrict__ xh,
-                                                            const float *__restrict__ xinv, float *__restrict__ y,
-                                                            int M, int N, int K, int Kp, int G, int row_bytes) {
-    constexpr int BN = 32 * WN;
-    constexpr int WStage = kWSlots * kBM * 4;
-    constexpr int StageBytes = WStage + BN * 128;
-    constexpr int P = 5 + WN;  // DMAs per wave per step
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = blockIdx.x * kBM, n0 = blockIdx.y * BN;
-    if constexpr (GT != 0) G = GT;
-    const int gb = 4 + G / 2;
-    const int groups = (K + G - 1) / G;
-    const int steps = Kp / kStepK;
-
-    const __amdgpu_buffer_rsrc_t wr = make_rsrc(w + static_cast<size_t>(m0) * row_bytes,
-                                                static_cast<size_t>(M - m0) * row_bytes);
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(xh + static_cast<size_t>(n0) * Kp,
-                                                static_cast<size_t>(N - n0) * Kp * 2);
-    int wvo[5], wslot[5];
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-        const int i = 5 * wave + q;
-        wslot[q] = i >> 1;
-        wvo[q] = (64 * (i & 1) + lane) * row_bytes;
-    }
-    int xvo[WN];
-#pragma unroll
-    for (int q = 0; q < WN; ++q) {
-        const int p = 64 * (WN * wave + q) + lane;
-        const int r = p >> 3, c = (p & 7) ^ ((r >> 1) & 7);
-        xvo[q] = r * Kp * 2 + 16 * c;
-    }
-    // G = 64: both halves of step s lie in group s, so a slot's offset is
-    // 36 * s plus a constant of the slot
-    int wconst[5];
-#pragma unroll
-    for (int q = 0; q < 5; ++q) wconst[q] = w_slot_offset<GT>(wslot[q], 0, G, gb, groups);
-    auto issue = [&](int s) {
-        int wso[5];
-        if constexpr (GT == 64) {
-            const int base = gb * min(s, groups - 1);
-#pragma unroll
-            for (int q = 0; q < 5; ++q) wso[q] = base + wconst[q];
-        } else {
-#pragma unroll
-            for (int q = 0; q < 5; ++q) wso[q] = w_slot_offset<GT>(wslot[q], s, G, gb, groups);
-        }
-        issue_step2(wr, xr, smem + (s % S) * StageBytes, wvo, wso, xvo, WN, s * kStepK * 2, WStage, wave);
-    };
-
-    f16x acc[WN];
-#pragma unroll
-    for (int j = 0; j < WN; ++j) acc[j] = f16x{};
-    const int li = lane & 31, kq = lane >> 5;
-    const int row = 32 * wave + li;
-    // LDS read offsets within a stage (bytes)
-    int xro[4][WN];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) {
-            const int r = 32 * j + li;
-            xro[kk][j] = WStage + 16 * (8 * r + ((2 * kk + kq) ^ ((r >> 1) & 7)));
-        }
-
-#pragma unroll
-    for (int s = 0; s < S - 1; ++s) issue(s);
-    for (int s = 0; s < steps; ++s) {
-        wait_vm((S - 2) * P);  // this wave's part of step s has landed
-        lds_barrier();         // every wave's part has; step s - 1's slot is free
-        issue(s + S - 1);      // (past the last step: never consumed)
-        const unsigned char *st = smem + (s % S) * StageBytes;
-        const unsigned *ws = reinterpret_cast<const unsigned *>(st);
-        const unsigned hd0 = ws[row], hd1 = ws[kBM + row];
-        unsigned c[4];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) c[kk] = ws[(2 + 4 * (kk >> 1) + 2 * (kk & 1) + kq) * kBM + row];
-        h8 b[4][WN];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-            for (int j = 0; j < WN; ++j) b[kk][j] = *reinterpret_cast<const h8 *>(st + xro[kk][j]);
-        const bool v0 = (s * kStepK) / G < groups, v1 = (s * kStepK + 32) / G < groups;
-        const float s0 = v0 ? half_bits_f(hd0) : 0.f;
-        const float s1 = v1 ? half_bits_f(hd1) : 0.f;
-        const float z0 = v0 ? -(half_bits_f(hd0 >> 16) * s0) : 0.f;
-        const float z1 = v1 ? -(half_bits_f(hd1 >> 16) * s1) : 0.f;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const h8 a = kk < 2 ? dequant8(c[kk], s0, z0) : dequant8(c[kk], s1, z1);
-#pragma unroll
-            for (int j = 0; j < WN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[kk][j], acc[j], 0, 0, 0);
-        }
-    }
-    wait_vm(0);
-
-    // epilogue: lane holds rows (r/4)*8 + (lane/32)*4 + r%4 of column lane%32
-#pragma unroll
-    for (int j = 0; j < WN; ++j) {
-        const int n = n0 + 32 * j + li;
-        if (n >= N) continue;
-        const float sc = xinv[n];
-        float *yc = y + static_cast<size_t>(n) * M;
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            const int m = m0 + 32 * wave + 8 * r4 + 4 * kq;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (m + q < M) yc[m + q] = acc[j][4 * r4 + q] * sc;
-        }
-    }
-}
-
-// ---- 4. G = 64: W straight into registers
-//   At G = 64 a step's 64 elements of a row are one group: 36 contiguous bytes
-//   [scale | zero | 32 code bytes] at 36 s. Lane (row, half h) loads the group
-//   header and the 16 code bytes of its half into VGPRs, S - 1 steps ahead, so W
-//   never passes through LDS (measured: the dword-granular W staging of
-//   i4_matmul_mfma2 was 40% of its time). X is staged as in i4_matmul_mfma2.
+// ---- 2. W straight into registers
+//   Lane (row, half h) takes 32 elements of its row per step: they lie in one group (G % 32 == 0),
+//   so a 4-byte load of its header and a 16-byte load of their codes, S - 1 steps ahead, bring
+//   them into VGPRs and W never passes through LDS. (W staged through LDS a dword at a time, as
+//   group sizes other than 64 used to be, took twice the time: 9728x2560 at G = 128 and 128 /
+//   512 / 3001 tokens 45 / 80 / 358 us per call against 25 / 47 / 210; at G = 64 a step's offsets are
+//   one scalar, at other sizes a select per half.)
+//   X: BN rows x 128 B of fp16 a step by DMA into a ring of S stages; 16-byte chunk c of token
+//   row r is stored at position c ^ ((r >> 1) & 7). A ds_read_b128 is served 16 lanes at a time,
+//   one 256-byte bank sweep: the 16 rows a group reads differ in (r & 1, chunk), so they cover
+//   the sweep once (no bank conflicts).
 //   The loop is unrolled by S so that every register slot index is a
 //   constant; steps past the last are loaded (never consumed) and not
 //   computed, which keeps every wait one constant s_waitcnt.
-//   The A operands are dequantized with packed fp16 arithmetic (dequant8_pk), which
-//   leaves a code dword's elements in k-slot order (0, 4, 1, 5, 2, 6, 3, 7); X comes
-//   from x_to_f16<true> in the same order, so both operands agree slot for slot.
+//   At G = 64 (PK) the A operands are dequantized with packed fp16 arithmetic (dequant8_pk),
+//   which leaves a code dword's elements in k-slot order (0, 4, 1, 5, 2, 6, 3, 7); X comes
+//   from x_to_f16<true> in the same order, so both operands agree slot for slot. Other group
+//   sizes keep the fp32 dequantization with its one rounding (dequant8) and X's natural order.
 //   Y leaves in 16-byte stores (4 rows of a token) where M % 4 == 0 and y is 16-byte
 //   aligned: four times fewer store instructions than one float each, which took
 //   the 512-token call from 48 to 39 us on MI355X (the output is 20 MB there).
@@ -669,11 +342,13 @@ __device__ __forceinline__ void issue_x(__amdgpu_buffer_rsrc_t xr, unsigned char
                 xr, (__attribute__((address_space(3))) void *)(st + 1024 * (d0 + q)), 16, xvo[q], xso, 0, 0);
 }
 
-template <int WN, int S, int NWV>
-__global__ __launch_bounds__(64 * NWV) void i4_matmul_g64(const uint8_t *__restrict__ w,
-                                                          const _Float16 *__restrict__ xh,
-                                                          const float *__restrict__ xinv, float *__restrict__ y, int M,
-                                                          int N, int K, int Kp, int row_bytes, int vec_y) {
+template <int GT, int WN, int S, int NWV>
+__global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__restrict__ w,
+                                                             const _Float16 *__restrict__ xh,
+                                                             const float *__restrict__ xinv, float *__restrict__ y,
+                                                             int M, int N, int K, int Kp, int G, int row_bytes,
+                                                             int vec_y) {
+    constexpr bool PK = GT == 64;  // packed-fp16 dequantization, X in its k-slot order
     constexpr int BN = 32 * WN;
     constexpr int BM = 32 * NWV;
     constexpr int XStage = BN * 128;
@@ -681,21 +356,22 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_g64(const uint8_t *__restr
     // them, the others XA. P: this wave's loads per step (W 4 + 16 bytes, its X DMAs).
     constexpr int XA = 4 * WN / NWV, XR = 4 * WN % NWV;
     constexpr int XD = XA + (XR ? 1 : 0);
-    constexpr int kGroupBytes = 36;
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-    const int groups = (K + 63) / 64;
-    const int steps = Kp / kStepK;  // = groups
+    if constexpr (GT != 0) G = GT;
+    const int gb = 4 + G / 2;
+    const int groups = (K + G - 1) / G;
+    const int steps = Kp / kStepK;
 
     const __amdgpu_buffer_rsrc_t wr = make_rsrc(w + static_cast<size_t>(m0) * row_bytes,
                                                 static_cast<size_t>(M - m0) * row_bytes);
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(xh + static_cast<size_t>(n0) * Kp,
                                                 static_cast<size_t>(N - n0) * Kp * 2);
-    // Lane (row li, half h) takes elements 32 h .. 32 h + 31 of every step: the group header
-    // and code bytes 16 h .. 16 h + 15; MFMA k-slot 8 h + p of k-block kk holds element
-    // 32 h + 8 kk + e, p = pk_slot(e), on the A (W) and the B (X) side.
+    // Lane (row li, half h) takes elements 32 h .. 32 h + 31 of every step: the header of their group
+    // (G % 32 == 0: they lie in one) and their 16 code bytes; MFMA k-slot 8 h + p of k-block kk
+    // holds element 32 h + 8 kk + e, p = pk_slot(e) (PK) or e, on the A (W) and the B (X) side.
     const int li = lane & 31, h = lane >> 5;
     const int wvo = (32 * wave + li) * row_bytes;
     const int nx = XA + (wave < XR ? 1 : 0), d0 = XA * wave + min(wave, XR);
@@ -720,9 +396,16 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_g64(const uint8_t *__restr
     u4v cd[S];
     auto issue = [&](auto uc, int s) {  // step s into register slot and X stage u = s % S
         constexpr int u = decltype(uc)::value;
-        const int so = kGroupBytes * min(s, groups - 1);  // (past the last step: in-row bytes, never used)
-        hd[u] = __builtin_amdgcn_raw_buffer_load_b32(wr, wvo, so, 0);
-        cd[u] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(wr, wvo + 4 + 16 * h, so, 0));
+        if constexpr (GT == 64) {
+            const int so = 36 * min(s, groups - 1);  // (past the last step: in-row bytes, never used)
+            hd[u] = __builtin_amdgcn_raw_buffer_load_b32(wr, wvo, so, 0);
+            cd[u] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(wr, wvo + 4 + 16 * h, so, 0));
+        } else {
+            const HalfOffsets o = half_offsets(s, G, gb, groups);
+            hd[u] = __builtin_amdgcn_raw_buffer_load_b32(wr, wvo + (h ? o.hdr[1] : o.hdr[0]), 0, 0);
+            cd[u] = __builtin_bit_cast(
+                u4v, __builtin_amdgcn_raw_buffer_load_b128(wr, wvo + (h ? o.code[1] : o.code[0]), 0, 0));
+        }
         issue_x<XD>(xr, smem + u * XStage, xvo, nx, d0, s * kStepK * 2);
     };
     f16x acc[WN];
@@ -733,13 +416,24 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_g64(const uint8_t *__restr
         constexpr int u = decltype(uc)::value;
         const unsigned char *st = smem + u * XStage;
         hf2 s2, c2;
-        pk_header(hd[u], s2, c2);
+        float fs, fz;
+        if constexpr (PK) {
+            pk_header(hd[u], s2, c2);
+        } else {
+            fs = half_bits_f(hd[u]);
+            fz = -(half_bits_f(hd[u] >> 16) * fs);
+            opaque_f32(fs, fz);
+        }
 #pragma unroll
         for (int kk = k0; kk < k1; ++kk) {
             h8 b[WN];
 #pragma unroll
             for (int j = 0; j < WN; ++j) b[j] = *reinterpret_cast<const h8 *>(st + xro[kk][j]);
-            const h8 a = dequant8_pk(cd[u][kk], s2, c2, pkc);
+            h8 a;
+            if constexpr (PK)
+                a = dequant8_pk(cd[u][kk], s2, c2, pkc);
+            else
+                a = dequant8(cd[u][kk], fs, fz);
 #pragma unroll
             for (int j = 0; j < WN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[j], acc[j], 0, 0, 0);
         }
@@ -807,7 +501,7 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_g64(const uint8_t *__restr
     }
 }
 
-// ---- 5. Few tokens (N <= 32, G = 64): one launch
+// ---- 3. Few tokens (N <= 32, G = 64): one launch
 //   A kernel launch costs a few microseconds on this GPU whatever it does, so at a few
 //   tokens a separate X conversion pass would cost as much as the GEMM. Here every
 //   workgroup converts the X it needs itself. The grid is (128-row tile) x (K slice):
@@ -1065,61 +759,22 @@ int raise_lds_limit(const void *fn, size_t &limit) {
     return kOk;
 }
 
-template <int WM, int WN, int GT>
-int launch_tiles(const uint8_t *w, const _Float16 *xh, const float *xinv, float *y, int M, int N, int K, int Kp, int G,
-                 int rb, hipStream_t stream) {
-    constexpr int BM = 128 * WM, BN = 32 * WN;
-    constexpr int stage = kWStage1 * WM + BN * 128;
-    const int S = std::max(2, std::min(4, (80 * 1024) / stage));  // ring depth within 80 KB of LDS
-    const size_t lds = static_cast<size_t>(S) * stage;
-    static size_t limit = 0;  // dynamic LDS the kernel may take (0: not raised from the default 64 KB yet)
-    if (lds > 64 * 1024 && limit == 0) {
-        // what the CU's 160 KB leaves beside the kernel's static LDS
-        const void *fn = reinterpret_cast<const void *>(i4_matmul_mfma<WM, WN, GT>);
-        if (raise_lds_limit(fn, limit) != kOk) return kLaunchFailed;
-    }
-    if (lds > 64 * 1024 && lds > limit) return kTooLarge;
-    const dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN);
-    hipLaunchKernelGGL((i4_matmul_mfma<WM, WN, GT>), grid, dim3(kThreads), lds, stream, w, xh, xinv, y, M, N, K, Kp, G,
-                       rb, S);
-    return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
-}
-
-template <int WN, int GT, int S>
-int launch_tiles2(const uint8_t *w, const _Float16 *xh, const float *xinv, float *y, int M, int N, int K, int Kp, int G,
+template <int GT, int WN, int S, int NWV>
+int launch_direct(const uint8_t *w, const _Float16 *xh, const float *xinv, float *y, int M, int N, int K, int Kp, int G,
                   int rb, hipStream_t stream) {
-    constexpr int BN = 32 * WN;
-    const size_t lds = static_cast<size_t>(S) * (kWSlots * kBM * 4 + BN * 128);
-    static size_t limit = 0;
-    if (lds > 64 * 1024 && limit == 0) {
-        const void *fn = reinterpret_cast<const void *>(i4_matmul_mfma2<WN, GT, S>);
-        if (raise_lds_limit(fn, limit) != kOk) return kLaunchFailed;
-    }
-    if (lds > 64 * 1024 && lds > limit) return kTooLarge;
-    // row offsets of the 128 staged rows and token-row offsets must fit the 32-bit DMA offsets
-    if (static_cast<size_t>(kBM) * rb + static_cast<size_t>(Kp) * 2 >= (1ull << 31)) return kTooLarge;
-    const dim3 grid((M + kBM - 1) / kBM, (N + BN - 1) / BN);
-    hipLaunchKernelGGL((i4_matmul_mfma2<WN, GT, S>), grid, dim3(kThreads), lds, stream, w, xh, xinv, y, M, N, K, Kp, G,
-                       rb);
-    return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
-}
-
-template <int WN, int S, int NWV>
-int launch_g64(const uint8_t *w, const _Float16 *xh, const float *xinv, float *y, int M, int N, int K, int Kp, int rb,
-               hipStream_t stream) {
     constexpr int BN = 32 * WN, BM = 32 * NWV;
     const size_t lds = static_cast<size_t>(S) * BN * 128;
     static size_t limit = 0;
     if (lds > 64 * 1024 && limit == 0) {
-        const void *fn = reinterpret_cast<const void *>(i4_matmul_g64<WN, S, NWV>);
+        const void *fn = reinterpret_cast<const void *>(i4_matmul_direct<GT, WN, S, NWV>);
         if (raise_lds_limit(fn, limit) != kOk) return kLaunchFailed;
     }
     if (lds > 64 * 1024 && lds > limit) return kTooLarge;
     if (static_cast<size_t>(BM) * rb + static_cast<size_t>(Kp) * 2 * BN >= (1ull << 31)) return kTooLarge;
     const dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN);
     const int vec_y = M % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
-    hipLaunchKernelGGL((i4_matmul_g64<WN, S, NWV>), grid, dim3(64 * NWV), lds, stream, w, xh, xinv, y, M, N, K, Kp,
-                       rb, vec_y);
+    hipLaunchKernelGGL((i4_matmul_direct<GT, WN, S, NWV>), grid, dim3(64 * NWV), lds, stream, w, xh, xinv, y, M, N, K,
+                       Kp, G, rb, vec_y);
     return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
 }
 
@@ -1221,18 +876,13 @@ int matmul_mfma(const uint8_t *w, const float *x, float *y, int M, int K, int N,
     _Float16 *xh = reinterpret_cast<_Float16 *>(ws);
     float *xinv = reinterpret_cast<float *>(ws + xh_bytes);
     const int ikp = static_cast<int>(Kp), irb = static_cast<int>(rb);
-    const int wn = pick_wn(N);
-    // The G = 64 kernel (packed-fp16 dequantization) takes X in its k-slot order; the other
-    // kernels in natural order. Its workgroups address 32 NWV rows and 32 WN token rows of X
-    // with 32-bit offsets.
-    const int g64_bm = wn == 1 ? 32 : wn == 2 ? 128 : 256;
-    const bool g64 = group_size == 64 && static_cast<size_t>(g64_bm) * rb + Kp * 2 * 32 * wn < (1ull << 31);
-    launch_x_to_f16(g64, x, K, ikp, N, xh, xinv, stream);
+    launch_x_to_f16(group_size == 64, x, K, ikp, N, xh, xinv, stream);
     if (hipGetLastError() != hipSuccess) return kLaunchFailed;
-    int st;
-    if (g64) {
-        // one-wave workgroups of 32 rows for a single token block: four times
-        // the workgroups (304 at 9728 rows), each with a wave-private X ring
+    const auto tiles = [&](auto gc) {
+        constexpr int GT = decltype(gc)::value;
+        const int wn = pick_wn(N);
+        // one-wave workgroups of 32 rows for a single token block: four times the workgroups (304 at
+        // 9728 rows), each with a wave-private X ring
         // Tiles measured on MI355X at 9728x2560 (512 / 128 tokens): 128 x 96 52.9 / 33.0 us,
         // 128 x 64 57.9 / 27.7, 128 x 128 58.7 / 38.9; two or more row blocks per wave
         // (256 x 96, 256 x 64, 128 x 96 over 2 waves, ...) 66-82 / 40-72; and staging W
@@ -1245,28 +895,14 @@ int matmul_mfma(const uint8_t *w, const float *x, float *y, int M, int K, int N,
         // 45.7-46.4; a 2-step ring: 60; the token tiles of a row tile on one XCD: no change).
         // At 128 tokens the 4-step ring of 4 waves stays (3 steps: 26.2 us, 2: 41.1, 128 x 32
         // tiles: 25.2, 256 x 32 tiles of 8 waves: 34.3, against 24.0).
-        return wn == 1   ? launch_g64<1, 4, 1>(w, xh, xinv, y, M, N, K, ikp, irb, stream)
-               : wn == 2 ? launch_g64<2, 4, 4>(w, xh, xinv, y, M, N, K, ikp, irb, stream)
-                         : launch_g64<3, 3, 8>(w, xh, xinv, y, M, N, K, ikp, irb, stream);
-    }
-    if (group_size == 64) {
-        st = wn == 1   ? launch_tiles2<1, 64, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream)
-             : wn == 2 ? launch_tiles2<2, 64, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream)
-                       : launch_tiles2<3, 64, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-    } else {
-        st = wn == 1   ? launch_tiles2<1, 0, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream)
-             : wn == 2 ? launch_tiles2<2, 0, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream)
-                       : launch_tiles2<3, 0, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-    }
-    if (st != kTooLarge) return st;
-    if (group_size == 64) {
-        if (wn == 1) return launch_tiles<1, 1, 64>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-        if (wn == 2) return launch_tiles<1, 2, 64>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-        return launch_tiles<1, 3, 64>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-    }
-    if (wn == 1) return launch_tiles<1, 1, 0>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-    if (wn == 2) return launch_tiles<1, 2, 0>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
-    return launch_tiles<1, 3, 0>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
+        const int st = wn == 1 ? static_cast<int>(kTooLarge)
+                       : wn == 2
+                           ? launch_direct<GT, 2, 4, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream)
+                           : launch_direct<GT, 3, 3, 8>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
+        if (st != kTooLarge) return st;  // (rows whose tile passes the 32-bit offsets: the smallest tile)
+        return launch_direct<GT, 1, 4, 1>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
+    };
+    return group_size == 64 ? tiles(std::integral_constant<int, 64>{}) : tiles(std::integral_constant<int, 0>{});
 }
 
 // ---- allocation-free variant --------------------------------------------------------------
@@ -1356,7 +992,8 @@ int launch_i4_matmul(const uint8_t *w, const float *x, float *y, int M, int K, i
     void *ws = nullptr;
     const int st = scratch_prefill(stream, prefill_scratch_bytes(K, N), &ws);  // the stream's (or scope's) buffer
     if (st != kOk) return st;
-    return matmul_mfma(w, x, y, M, K, N, group_size, static_cast<unsigned char *>(ws), stream);
+    const int mst = matmul_mfma(w, x, y, M, K, N, group_size, static_cast<unsigned char *>(ws), stream);
+    return mst == kTooLarge ? matmul_by_columns(w, x, y, M, K, N, group_size, stream) : mst;
 }
 
 }  // namespace tqhip
