@@ -48,3 +48,24 @@ def test_other_group_sizes(gpu, orc, M, K, N, G):
         assert fp16_operand_bound_ok(got, want, orc, w, x, M, K, N, G)
     else:
         assert rel_l2(got, want) <= 2e-3
+
+
+# every count of steps left over after the rounds of the tiles' rings (3 and 4 steps of 64), from
+# fewer steps than a ring holds, on grids of several workgroups per CU and repeated: a step whose
+# activations were not waited for shows only now and then
+@pytest.mark.parametrize("steps", [1, 2, 3, 5, 6, 7, 15])
+@pytest.mark.parametrize("N,G", [(40, 64), (128, 64), (20, 128), (128, 128), (200, 64), (200, 32)])
+def test_steps_left_over(gpu, orc, steps, N, G):
+    M, K = 9728, 64 * steps
+    w, x = gpu.synth_i4(M, K, G, seed=steps + N), gpu.synth_normal(K * N, seed=steps)
+    want = orc.matmul_i4(w, x, M, K, N, G, threads=16)
+    dw, dx, dy = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(4 * M * N)
+    first = None
+    for _ in range(8):
+        gpu.lib().tqhip_memset(dy.ptr, 0xFF, 4 * M * N)
+        gpu.matmul_i4_dev(dw, dx, dy, M, K, N, G)
+        gpu.synchronize()
+        got = dy.download(np.float32, M * N)
+        first = got if first is None else first
+        assert np.array_equal(got.view(np.uint32), first.view(np.uint32))
+    assert rel_l2(first, want) <= 2e-3

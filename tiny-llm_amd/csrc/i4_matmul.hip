@@ -318,8 +318,8 @@ __device__ __forceinline__ HalfOffsets half_offsets(int s, int G, int gb, int gr
 //   one 256-byte bank sweep: the 16 rows a group reads differ in (r & 1, chunk), so they cover
 //   the sweep once (no bank conflicts).
 //   The loop is unrolled by S so that every register slot index is a
-//   constant; steps past the last are loaded (never consumed) and not
-//   computed, which keeps every wait one constant s_waitcnt.
+//   constant; its last round loads steps past the last (never consumed),
+//   which keeps every wait in it one constant s_waitcnt.
 //   At G = 64 (PK) the A operands are dequantized with packed fp16 arithmetic (dequant8_pk),
 //   which leaves a code dword's elements in k-slot order (0, 4, 1, 5, 2, 6, 3, 7); X comes
 //   from x_to_f16<true> in the same order, so both operands agree slot for slot. Other group
@@ -438,46 +438,48 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__re
             for (int j = 0; j < WN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[j], acc[j], 0, 0, 0);
         }
     };
-    // full: the step is below `steps`. Its loads of step s + S - 1 go in between the first and
-    // the last two k-blocks' MFMAs (program order; no branch), so that a wave stalled on a full
-    // memory pipeline has MFMAs in flight.
-    auto round_step = [&](auto uc, int s, auto full) {
+    // One step of a full round. Its loads of step s + S - 1 go in between the first and the last two
+    // k-blocks' MFMAs (program order; no branch), so that a wave stalled on a full memory pipeline
+    // has MFMAs in flight.
+    auto round_step = [&](auto uc, int s) {
         constexpr int u = decltype(uc)::value;
         if (XR == 0 || wave < XR)  // this wave's loads of step s have landed
             wait_vm((S - 2) * (2 + XD));
         else
             wait_vm((S - 2) * (2 + XA));
         lds_barrier();  // every wave's X part has; step s - 1's stage is free
-        if constexpr (decltype(full)::value) {
-            compute(uc, 0, 2);
-            issue(std::integral_constant<int, (u + S - 1) % S>{}, s + S - 1);
-            compute(uc, 2, 4);
-        } else {
-            issue(std::integral_constant<int, (u + S - 1) % S>{}, s + S - 1);
-            if (s < steps) compute(uc, 0, 4);
-        }
+        compute(uc, 0, 2);
+        issue(std::integral_constant<int, (u + S - 1) % S>{}, s + S - 1);
+        compute(uc, 2, 4);
     };
 
+    // (the sched_barriers keep each step's loads together: the waits count whole steps)
     issue(std::integral_constant<int, 0>{}, 0);
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (S > 2) issue(std::integral_constant<int, 1>{}, 1);
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (S > 3) issue(std::integral_constant<int, 2>{}, 2);
+    __builtin_amdgcn_sched_barrier(0);
     static_assert(S >= 2 && S <= 4, "register slots 0..3");
-    const std::true_type full;
-    const std::false_type tail;
     int s0 = 0;
     for (; s0 + S <= steps; s0 += S) {
-        round_step(std::integral_constant<int, 0>{}, s0, full);
-        round_step(std::integral_constant<int, 1>{}, s0 + 1, full);
-        if constexpr (S > 2) round_step(std::integral_constant<int, 2>{}, s0 + 2, full);
-        if constexpr (S > 3) round_step(std::integral_constant<int, 3>{}, s0 + 3, full);
+        round_step(std::integral_constant<int, 0>{}, s0);
+        round_step(std::integral_constant<int, 1>{}, s0 + 1);
+        if constexpr (S > 2) round_step(std::integral_constant<int, 2>{}, s0 + 2);
+        if constexpr (S > 3) round_step(std::integral_constant<int, 3>{}, s0 + 3);
     }
-    if (s0 < steps) {
-        round_step(std::integral_constant<int, 0>{}, s0, tail);
-        round_step(std::integral_constant<int, 1>{}, s0 + 1, tail);
-        if constexpr (S > 2) round_step(std::integral_constant<int, 2>{}, s0 + 2, tail);
-        if constexpr (S > 3) round_step(std::integral_constant<int, 3>{}, s0 + 3, tail);
-    }
+    // The last steps % S steps: all of their loads are under way, so one wait for everything and no
+    // more loads. (Issuing loads here to keep the constant waits would not do: nothing reads the
+    // codes that they bring, so the compiler drops those loads and the waits then count too few.)
     wait_vm(0);
+    lds_barrier();
+    if (s0 < steps) compute(std::integral_constant<int, 0>{}, 0, 4);
+    if constexpr (S > 2) {
+        if (s0 + 1 < steps) compute(std::integral_constant<int, 1>{}, 0, 4);
+    }
+    if constexpr (S > 3) {
+        if (s0 + 2 < steps) compute(std::integral_constant<int, 2>{}, 0, 4);
+    }
 
     // epilogue: lane holds rows (r/4)*8 + (lane/32)*4 + r%4 of column lane%32
 #pragma unroll
