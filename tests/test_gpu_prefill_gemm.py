@@ -69,3 +69,54 @@ def test_steps_left_over(gpu, orc, steps, N, G):
         first = got if first is None else first
         assert np.array_equal(got.view(np.uint32), first.view(np.uint32))
     assert rel_l2(first, want) <= 2e-3
+
+
+# K slices (kSplitParts, kSplitSeq): few tiles and many steps, with slices of unequal step counts, at
+# the tile edges; both tiles that are split, both dequantizations. The device entry point adds the
+# slices' partials, the allocation-free one runs the slices one after the other: the same bits,
+# and the same again on every repeat (whichever slice arrives last).
+@pytest.mark.parametrize("M,K,N,G", [(128, 9728, 40, 64), (129, 4864, 65, 64), (896, 4864, 128, 64), (1, 4160, 33, 64),
+                                     (1000, 2560, 256, 128), (40, 9728, 32, 128), (513, 4900, 1, 32),
+                                     (4096, 2560, 16, 256), (2560, 9728, 200, 96)])
+def test_k_slices(gpu, orc, M, K, N, G):
+    w, x = gpu.synth_i4(M, K, G, seed=M + N), gpu.synth_normal(K * N, seed=K)
+    want = orc.matmul_i4(w, x, M, K, N, G, threads=16)
+    dw, dx, dy = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(4 * M * N)
+    outs = []
+    for i in range(7):
+        gpu.lib().tqhip_memset(dy.ptr, 0xFF, 4 * M * N)
+        if i < 6:
+            gpu.matmul_i4_dev(dw, dx, dy, M, K, N, G)
+        else:
+            assert gpu.matmul_i4_noalloc_dev(dw, dx, dy, M, K, N, G) == gpu.OK
+        gpu.synchronize()
+        outs.append(dy.download(np.float32, M * N))
+        assert np.array_equal(outs[i].view(np.uint32), outs[0].view(np.uint32)), i
+    if M * N < 64:
+        assert fp16_operand_bound_ok(outs[0], want, orc, w, x, M, K, N, G)
+    else:
+        assert rel_l2(outs[0], want) <= 2e-3
+
+
+def test_k_slices_in_a_captured_graph(gpu, orc):
+    """Split calls captured into an op graph: replays with new activations, eager work and
+    synchronisations between them give the eager bits (the counters are zero after every replay)."""
+    shapes = [(896, 4864, 48, 64), (1024, 2560, 20, 128)]
+    bufs = [(gpu.DeviceBuffer.from_array(gpu.synth_i4(M, K, G, seed=M)), gpu.DeviceBuffer(4 * K * N),
+             gpu.DeviceBuffer(4 * M * N)) for M, K, N, G in shapes]
+    ops = [gpu.Op(gpu.OP_I4_MATMUL, w.ptr, x.ptr, y.ptr, M, K, N, G) for (w, x, y), (M, K, N, G) in zip(bufs, shapes)]
+    stream = gpu.Stream()
+    graph = gpu.OpsGraph(ops, stream)
+    try:
+        for rep in range(4):
+            for (_, x, _), (M, K, N, _) in zip(bufs, shapes):
+                x.upload(gpu.synth_normal(K * N, seed=rep + M))
+            graph.launch()
+            stream.synchronize()
+            got = [y.download(np.float32, M * N) for (_, _, y), (M, _, N, _) in zip(bufs, shapes)]
+            gpu.run_ops(ops, 1)
+            gpu.synchronize()
+            for g, (_, _, y), (M, _, N, _) in zip(got, bufs, shapes):
+                assert np.array_equal(g.view(np.uint32), y.download(np.float32, M * N).view(np.uint32)), rep
+    finally:
+        graph.close()

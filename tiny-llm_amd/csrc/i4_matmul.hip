@@ -306,6 +306,98 @@ __device__ __forceinline__ HalfOffsets half_offsets(int s, int G, int gb, int gr
     return o;
 }
 
+// ---- K slices of a tile
+//   A grid of few tiles leaves most CUs idle, so K is then cut into KS slices of whole steps, one
+//   workgroup each (kSplitParts): a workgroup stores its partial product, the last of a tile to
+//   arrive adds the KS partials in slice order (the same bits whatever the arrival order) and
+//   stores Y. kSplitSeq gives the same bits with one workgroup per tile and no partials, for calls
+//   that may not allocate them.
+constexpr int kSplitNone = 0, kSplitParts = 1, kSplitSeq = 2;
+constexpr int kDeviceScope = 16;  // buffer cache policy: sc1 (device-scope coherent)
+constexpr int kL1Bypass = 1;      // buffer cache policy: sc0 (misses in the CU's L1, served by the XCD's L2)
+constexpr int kXccSlots = 14;     // slices whose writer's XCD the arrival counter carries
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+//   Partials are [tile][slice][wave][token block][float4][lane] (the MFMA's register order: every
+//   store and load instruction moves 1 KB in one piece), written at device scope (sc1: through this
+//   XCD's L2 to the level where all XCDs meet), so a store that has completed is visible
+//   everywhere and the arrival counter (zero between launches: the last arrival resets it) needs
+//   no cache write-back or invalidation, both of which act on a whole L2. The counter add carries
+//   the writer's XCD (slices below kXccSlots): the last arrival reads a partial written on its own
+//   XCD from that L2 (which the write went through) and any other one at device scope.
+//   True for the last arrival, whose acc then holds the sum.
+template <int WN, int NWV>
+__device__ inline bool add_parts(f16x (&acc)[WN], float *part, unsigned long long *arrivals, int tile, int ks, int KS,
+                                 int wave, int lane) {
+    constexpr int kPart = 32 * NWV * 32 * WN;  // floats of one partial
+    constexpr int V = 4 * WN;                  // float4s of a lane
+    constexpr int B = V <= 4 ? 6 : V <= 8 ? 4 : 2;  // partials in flight at once (registers)
+    __shared__ int last_s;
+    __shared__ unsigned long long writers_s;
+    const int xcc = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 7;  // HW_REG_XCC_ID bits 0..3
+    const __amdgpu_buffer_rsrc_t pr =
+        make_rsrc(part + static_cast<size_t>(tile) * KS * kPart, static_cast<size_t>(KS) * kPart * sizeof(float));
+    const int lo = 16 * (64 * V * wave + lane);
+    f4v own[V];
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+            own[4 * j + r4] = f4v{acc[j][4 * r4], acc[j][4 * r4 + 1], acc[j][4 * r4 + 2], acc[j][4 * r4 + 3]};
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, own[v]), pr, lo + 4 * (ks * kPart) + 1024 * v, 0,
+                                               kDeviceScope);
+    wait_vm(0);       // this wave's partial stores have completed
+    __syncthreads();  // and every other wave's
+    if (threadIdx.x == 0) {
+        // bits 56..63: arrivals; bits 4 p .. 4 p + 3: 1 + the XCD of slice p's writer
+        const unsigned long long mine =
+            (1ull << 56) | (ks < kXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
+        const unsigned long long prev =
+            __hip_atomic_fetch_add(arrivals + tile, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = (prev >> 56) == static_cast<unsigned long long>(KS - 1);
+        if (last) __hip_atomic_store(arrivals + tile, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last_s = last;
+        writers_s = prev;
+    }
+    __syncthreads();
+    if (!last_s) return false;
+    const unsigned long long writers = writers_s;
+    f4v sum[V] = {};
+    for (int p0 = 0; p0 < KS; p0 += B) {
+        f4v v[B][V];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int p = min(p0 + u, KS - 1);
+            if (p == ks) continue;
+            const bool here = p < kXccSlots && ((writers >> (4 * p)) & 15) == static_cast<unsigned>(xcc + 1);
+            if (here) {
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    v[u][i] = __builtin_bit_cast(
+                        f4v, __builtin_amdgcn_raw_buffer_load_b128(pr, lo + 4 * (p * kPart) + 1024 * i, 0, kL1Bypass));
+            } else {
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    v[u][i] = __builtin_bit_cast(
+                        f4v, __builtin_amdgcn_raw_buffer_load_b128(pr, lo + 4 * (p * kPart) + 1024 * i, 0, kDeviceScope));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            if (p0 + u >= KS) break;
+#pragma unroll
+            for (int i = 0; i < V; ++i) sum[i] += p0 + u == ks ? own[i] : v[u][i];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = sum[4 * j + r / 4][r % 4];
+    return true;
+}
+
 // ---- 2. W straight into registers
 //   Lane (row, half h) takes 32 elements of its row per step: they lie in one group (G % 32 == 0),
 //   so a 4-byte load of its header and a 16-byte load of their codes, S - 1 steps ahead, bring
@@ -342,12 +434,13 @@ __device__ __forceinline__ void issue_x(__amdgpu_buffer_rsrc_t xr, unsigned char
                 xr, (__attribute__((address_space(3))) void *)(st + 1024 * (d0 + q)), 16, xvo[q], xso, 0, 0);
 }
 
-template <int GT, int WN, int S, int NWV>
+template <int GT, int WN, int S, int NWV, int SPLIT>
 __global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__restrict__ w,
                                                              const _Float16 *__restrict__ xh,
                                                              const float *__restrict__ xinv, float *__restrict__ y,
                                                              int M, int N, int K, int Kp, int G, int row_bytes,
-                                                             int vec_y) {
+                                                             int vec_y, int KS, float *__restrict__ part,
+                                                             unsigned long long *__restrict__ arrivals) {
     constexpr bool PK = GT == 64;  // packed-fp16 dequantization, X in its k-slot order
     constexpr int BN = 32 * WN;
     constexpr int BM = 32 * NWV;
@@ -359,7 +452,20 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__re
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
+    int tile = 0, ks = 0, m0, n0;
+    if constexpr (SPLIT == kSplitParts) {
+        // the slices of a tile are 8 workgroups apart, so with workgroups dealt to the 8 XCDs in
+        // turn they share one XCD
+        tile = (blockIdx.x / (8 * KS)) * 8 + (blockIdx.x & 7);
+        ks = (blockIdx.x >> 3) % KS;
+        const int mtiles = (M + BM - 1) / BM, nt = tile / mtiles;
+        m0 = (tile - nt * mtiles) * BM;
+        n0 = nt * BN;
+        if (n0 >= N) return;  // a padding tile (the tile count rounded up to 8)
+    } else {
+        m0 = blockIdx.x * BM;
+        n0 = blockIdx.y * BN;
+    }
     if constexpr (GT != 0) G = GT;
     const int gb = 4 + G / 2;
     const int groups = (K + G - 1) / G;
@@ -453,51 +559,83 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__re
         compute(uc, 2, 4);
     };
 
-    // (the sched_barriers keep each step's loads together: the waits count whole steps)
-    issue(std::integral_constant<int, 0>{}, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (S > 2) issue(std::integral_constant<int, 1>{}, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (S > 3) issue(std::integral_constant<int, 2>{}, 2);
-    __builtin_amdgcn_sched_barrier(0);
     static_assert(S >= 2 && S <= 4, "register slots 0..3");
-    int s0 = 0;
-    for (; s0 + S <= steps; s0 += S) {
-        round_step(std::integral_constant<int, 0>{}, s0);
-        round_step(std::integral_constant<int, 1>{}, s0 + 1);
-        if constexpr (S > 2) round_step(std::integral_constant<int, 2>{}, s0 + 2);
-        if constexpr (S > 3) round_step(std::integral_constant<int, 3>{}, s0 + 3);
+    // Steps sa .. sb - 1 into acc (slot u holds step sa + u modulo S).
+    // (the sched_barriers keep each step's loads together: the waits count whole steps)
+    auto run = [&](int sa, int sb) {
+        issue(std::integral_constant<int, 0>{}, sa);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (S > 2) issue(std::integral_constant<int, 1>{}, sa + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (S > 3) issue(std::integral_constant<int, 2>{}, sa + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        int s0 = sa;
+        for (; s0 + S <= sb; s0 += S) {
+            round_step(std::integral_constant<int, 0>{}, s0);
+            round_step(std::integral_constant<int, 1>{}, s0 + 1);
+            if constexpr (S > 2) round_step(std::integral_constant<int, 2>{}, s0 + 2);
+            if constexpr (S > 3) round_step(std::integral_constant<int, 3>{}, s0 + 3);
+        }
+        // The last (sb - sa) % S steps: all of their loads are under way, so one wait for everything
+        // and no more loads. (Issuing loads here to keep the constant waits would not do: nothing
+        // reads the codes that they bring, so the compiler drops those loads and the waits then
+        // count too few.)
+        wait_vm(0);
+        lds_barrier();
+        if (s0 < sb) compute(std::integral_constant<int, 0>{}, 0, 4);
+        if constexpr (S > 2) {
+            if (s0 + 1 < sb) compute(std::integral_constant<int, 1>{}, 0, 4);
+        }
+        if constexpr (S > 3) {
+            if (s0 + 2 < sb) compute(std::integral_constant<int, 2>{}, 0, 4);
+        }
+    };
+    // each token's scale, requested before the stores below (a load behind them waits for them)
+    float sc[WN];
+    const auto load_scales = [&]() {
+#pragma unroll
+        for (int j = 0; j < WN; ++j) sc[j] = xinv[min(n0 + 32 * j + li, N - 1)];
+    };
+    if constexpr (SPLIT == kSplitNone) {
+        run(0, steps);
+    } else if constexpr (SPLIT == kSplitParts) {
+        run((ks * steps) / KS, ((ks + 1) * steps) / KS);
+        if (!add_parts<WN, NWV>(acc, part, arrivals, tile, ks, KS, wave, lane)) return;
+    } else {
+        // every slice in this workgroup, added as add_parts adds them: the same bits without partials
+        f16x sum[WN];
+#pragma unroll
+        for (int j = 0; j < WN; ++j) sum[j] = f16x{};
+        for (int p = 0; p < KS; ++p) {
+            run((p * steps) / KS, ((p + 1) * steps) / KS);
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                sum[j] += acc[j];
+                acc[j] = f16x{};
+            }
+            lds_barrier();  // (every wave is done with the stages that the next slice's loads go to)
+        }
+#pragma unroll
+        for (int j = 0; j < WN; ++j) acc[j] = sum[j];
     }
-    // The last steps % S steps: all of their loads are under way, so one wait for everything and no
-    // more loads. (Issuing loads here to keep the constant waits would not do: nothing reads the
-    // codes that they bring, so the compiler drops those loads and the waits then count too few.)
-    wait_vm(0);
-    lds_barrier();
-    if (s0 < steps) compute(std::integral_constant<int, 0>{}, 0, 4);
-    if constexpr (S > 2) {
-        if (s0 + 1 < steps) compute(std::integral_constant<int, 1>{}, 0, 4);
-    }
-    if constexpr (S > 3) {
-        if (s0 + 2 < steps) compute(std::integral_constant<int, 2>{}, 0, 4);
-    }
+    load_scales();
 
     // epilogue: lane holds rows (r/4)*8 + (lane/32)*4 + r%4 of column lane%32
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
         const int n = n0 + 32 * j + li;
         if (n >= N) continue;
-        const float sc = xinv[n];
         float *yc = y + static_cast<size_t>(n) * M;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             const int m = m0 + 32 * wave + 8 * r4 + 4 * h;
             if (vec_y && m + 3 < M) {
-                *reinterpret_cast<float4 *>(yc + m) = make_float4(acc[j][4 * r4] * sc, acc[j][4 * r4 + 1] * sc,
-                                                                  acc[j][4 * r4 + 2] * sc, acc[j][4 * r4 + 3] * sc);
+                *reinterpret_cast<float4 *>(yc + m) = make_float4(acc[j][4 * r4] * sc[j], acc[j][4 * r4 + 1] * sc[j],
+                                                                  acc[j][4 * r4 + 2] * sc[j], acc[j][4 * r4 + 3] * sc[j]);
             } else {
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    if (m + q < M) yc[m + q] = acc[j][4 * r4 + q] * sc;
+                    if (m + q < M) yc[m + q] = acc[j][4 * r4 + q] * sc[j];
             }
         }
     }
@@ -533,11 +671,7 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__re
 //     last arrival resets it) carries each writer's XCD, so a partial written elsewhere is
 //     read at device scope instead.
 constexpr int kSkRows = 128;
-constexpr int kDeviceScope = 16;  // buffer cache policy: sc1 (device-scope coherent)
-constexpr int kL1Bypass = 1;      // buffer cache policy: sc0 (misses in the CU's L1, served by the XCD's L2)
-constexpr int kSkXccSlots = 14;   // slices whose writer's XCD the arrival counter carries
 constexpr int kSkReduceBatch = 6; // partials the last arrival has in flight at once
-typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kSkTile = kSkRows * 32;  // floats of one partial
 constexpr int kSkMaxSteps = 7;  // a row's slice (9 dwords a step) within one 64-lane DMA
 
@@ -664,7 +798,7 @@ __global__ __launch_bounds__(256) void i4_matmul_skinny(const uint8_t *__restric
     //    device scope (sc1: written through this XCD's L2 to the level where all XCDs meet),
     //    so a store that has completed is visible everywhere and the counter needs no cache
     //    write-back or invalidation (both act on a whole L2). The counter add carries the
-    //    writer's XCD (slices < kSkXccSlots): the last arrival reads a partial written on its
+    //    writer's XCD (slices < kXccSlots): the last arrival reads a partial written on its
     //    own XCD from that L2 (which the write went through) and any other one at device
     //    scope (its own L2 may hold an older copy of the line).
     const float iv = inv_s[li];
@@ -686,7 +820,7 @@ __global__ __launch_bounds__(256) void i4_matmul_skinny(const uint8_t *__restric
         if (threadIdx.x == 0) {
             // bits 56..63: arrivals; bits 4 p .. 4 p + 3: 1 + the XCD of slice p's writer
             const unsigned long long mine =
-                (1ull << 56) | (ks < kSkXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
+                (1ull << 56) | (ks < kXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
             const unsigned long long prev =
                 __hip_atomic_fetch_add(arrivals + tile, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const bool last = (prev >> 56) == static_cast<unsigned long long>(KS - 1);
@@ -708,7 +842,7 @@ __global__ __launch_bounds__(256) void i4_matmul_skinny(const uint8_t *__restric
         for (int u = 0; u < kSkReduceBatch; ++u) {
             const int p = min(p0 + u, KS - 1);
             if (p == ks) continue;
-            const bool here = p < kSkXccSlots && ((writers >> (4 * p)) & 15) == static_cast<unsigned>(xcc + 1);
+            const bool here = p < kXccSlots && ((writers >> (4 * p)) & 15) == static_cast<unsigned>(xcc + 1);
             if (here) {
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4)
@@ -761,22 +895,30 @@ int raise_lds_limit(const void *fn, size_t &limit) {
     return kOk;
 }
 
-template <int GT, int WN, int S, int NWV>
+// K slices of a call and where their partials go (part null: kSplitSeq).
+struct Slices {
+    int KS;
+    float *part;
+    unsigned long long *arrivals;
+};
+
+template <int GT, int WN, int S, int NWV, int SPLIT>
 int launch_direct(const uint8_t *w, const _Float16 *xh, const float *xinv, float *y, int M, int N, int K, int Kp, int G,
-                  int rb, hipStream_t stream) {
+                  int rb, const Slices &sl, hipStream_t stream) {
     constexpr int BN = 32 * WN, BM = 32 * NWV;
+    const auto kernel = i4_matmul_direct<GT, WN, S, NWV, SPLIT>;
     const size_t lds = static_cast<size_t>(S) * BN * 128;
     static size_t limit = 0;
     if (lds > 64 * 1024 && limit == 0) {
-        const void *fn = reinterpret_cast<const void *>(i4_matmul_direct<GT, WN, S, NWV>);
-        if (raise_lds_limit(fn, limit) != kOk) return kLaunchFailed;
+        if (raise_lds_limit(reinterpret_cast<const void *>(kernel), limit) != kOk) return kLaunchFailed;
     }
     if (lds > 64 * 1024 && lds > limit) return kTooLarge;
     if (static_cast<size_t>(BM) * rb + static_cast<size_t>(Kp) * 2 * BN >= (1ull << 31)) return kTooLarge;
-    const dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN);
+    dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN);
+    if (SPLIT == kSplitParts) grid = dim3((grid.x * grid.y + 7) / 8 * 8 * sl.KS);
     const int vec_y = M % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
-    hipLaunchKernelGGL((i4_matmul_direct<GT, WN, S, NWV>), grid, dim3(64 * NWV), lds, stream, w, xh, xinv, y, M, N, K,
-                       Kp, G, rb, vec_y);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NWV), lds, stream, w, xh, xinv, y, M, N, K, Kp, G, rb, vec_y, sl.KS,
+                       sl.part, sl.arrivals);
     return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
 }
 
@@ -826,11 +968,55 @@ int launch_skinny(const uint8_t *w, const float *x, float *y, int M, int K, int 
     return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
 }
 
-// Token blocks of 32 per wave (WN). Measured on MI355X at 9728x2560: one
-// block for <= 32 tokens, two for <= 128 (30.6 vs 38.2 us at 128 tokens),
-// three above (128-token tiles and two row blocks per wave were slower: fewer
-// workgroups, more registers).
-int pick_wn(int N) { return N <= 32 ? 1 : N <= 128 ? 2 : 3; }
+// A call's tile and K slices (KS > 1: one workgroup per tile and slice).
+enum TileKind { kTile32x32, kTile128x32, kTile128x64, kTile256x96 };
+struct TilePlan {
+    TileKind kind;
+    int KS;
+    size_t tiles, part_bytes;  // of a split call
+};
+
+// The plan with the least estimated time, from what a step of each tile takes on MI355X when a CU
+// holds one, two or n workgroups of it (us) and what the exchange of a split adds: stores, counter
+// and the last arrival's reads (16 or 32 KB a partial at 50-90 GB/s), and the partials' way through
+// memory (twice, 6 TB/s). It only has to rank. Measured against the choice of one tile per token
+// count without slices that it replaces (us per call, G = 64): 2560x9728 at 48 / 128 / 512 tokens
+// 65 / 72 / 122 -> 21 / 24 / 50; 1024x2560 at 128 / 512 20 / 34 -> 15 / 18; 4096x2560 at 256 33 -> 19.
+// The old choice where it was right: 9728x2560 at 128 (152 tiles: 21, with two to five slices 23-31)
+// and at 512 (256 x 96 tiles: 41, 128 x 64 49); 896x896 at 128 whole (14 steps: 10.6, with slices 14).
+// A function of the shape and the device alone: every entry point gives a call the same sums.
+TilePlan tile_plan(int M, int K, int N) {
+    const int steps = (K + kStepK - 1) / kStepK, cus = device_cu_count();
+    struct Tile {
+        TileKind kind;
+        int bm, bn;
+        float one, two, many;  // a step with one or two workgroups on the CU, and per workgroup with more
+        float split, part;     // a split, and each partial of a tile; split 0: not split
+    };
+    constexpr Tile kTiles[] = {{kTile32x32, 32, 32, 0.3f, 0.3f, 0.1f, 0.f, 0.f},
+                               {kTile128x32, 128, 32, 0.3f, 0.4f, 0.25f, 4.f, 0.25f},
+                               {kTile128x64, 128, 64, 0.4f, 0.6f, 0.42f, 4.f, 0.45f},
+                               {kTile256x96, 256, 96, 0.77f, 1.6f, 0.8f, 0.f, 0.f}};
+    constexpr int kMaxSlices = 32;
+    TilePlan best{};
+    float cost = 0.f;
+    for (const Tile &t : kTiles) {
+        // one token block: the 32-token tiles; more: the others (they share W loads among tokens)
+        if ((N <= 32) != (t.bn == 32)) continue;
+        const size_t tiles = static_cast<size_t>((M - 1) / t.bm + 1) * ((N - 1) / t.bn + 1);
+        for (int ks = 1; ks <= (t.split > 0.f ? std::min(kMaxSlices, steps) : 1); ++ks) {
+            const size_t n = (tiles * ks - 1) / cus + 1, bytes = ks > 1 ? tiles * ks * t.bm * t.bn * sizeof(float) : 0;
+            const float step = n == 1 ? t.one : n == 2 ? t.two : t.many * static_cast<float>(n);
+            const float c = static_cast<float>((steps - 1) / ks + 1) * step +
+                            (ks > 1 ? t.split + t.part * static_cast<float>(ks) + static_cast<float>(bytes) / 3e6f : 0.f);
+            if (best.tiles == 0 || c < cost) {
+                best = TilePlan{t.kind, ks, tiles, bytes};
+                cost = c;
+            }
+        }
+    }
+    return best;
+}
 
 // The MFMA path applies: a group size that is a multiple of 32 and byte offsets within 31 bits.
 bool mfma_applies(int M, int K, int N, int group_size) {
@@ -869,9 +1055,14 @@ void launch_x_to_f16(bool perm, const float *x, int K, int Kp, int N, _Float16 *
         launch_x_to_f16<false>(x, K, Kp, N, xh, xinv, stream);
 }
 
-// The MFMA path with X's fp16 copy and per-token scales at ws (prefill_scratch_bytes(K, N) bytes).
+// The partials of a split call follow X's copy in the workspace.
+size_t part_offset(int K, int N) { return (prefill_scratch_bytes(K, N) + 255) / 256 * 256; }
+
+// The MFMA path with X's fp16 copy and per-token scales at ws (prefill_scratch_bytes(K, N) bytes), and
+// with arrivals (tl.tiles counters, zero between launches) the partials of a split call after
+// them; arrivals null: its slices one after the other.
 int matmul_mfma(const uint8_t *w, const float *x, float *y, int M, int K, int N, int group_size, unsigned char *ws,
-                hipStream_t stream) {
+                const TilePlan &tl, unsigned long long *arrivals, hipStream_t stream) {
     const size_t rb = i4_row_bytes(K, group_size);
     const size_t Kp = (static_cast<size_t>(K) + kStepK - 1) / kStepK * kStepK;
     const size_t xh_bytes = (Kp * 2 * N + 255) / 256 * 256;
@@ -880,29 +1071,33 @@ int matmul_mfma(const uint8_t *w, const float *x, float *y, int M, int K, int N,
     const int ikp = static_cast<int>(Kp), irb = static_cast<int>(rb);
     launch_x_to_f16(group_size == 64, x, K, ikp, N, xh, xinv, stream);
     if (hipGetLastError() != hipSuccess) return kLaunchFailed;
+    const Slices sl{tl.KS, arrivals ? reinterpret_cast<float *>(ws + part_offset(K, N)) : nullptr, arrivals};
+    const auto go = [&](auto gc, auto wnc, auto sc, auto wvc) {
+        constexpr int GT = decltype(gc)::value, WN = decltype(wnc)::value, S = decltype(sc)::value,
+                      NWV = decltype(wvc)::value;
+        if constexpr (WN <= 2 && NWV == 4) {
+            if (tl.KS > 1 && sl.part)
+                return launch_direct<GT, WN, S, NWV, kSplitParts>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, sl,
+                                                                  stream);
+            if (tl.KS > 1)
+                return launch_direct<GT, WN, S, NWV, kSplitSeq>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, sl,
+                                                                stream);
+        }
+        return launch_direct<GT, WN, S, NWV, kSplitNone>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, sl, stream);
+    };
     const auto tiles = [&](auto gc) {
+        const std::integral_constant<int, 1> c1;
+        const std::integral_constant<int, 2> c2;
+        const std::integral_constant<int, 3> c3;
+        const std::integral_constant<int, 4> c4;
+        const std::integral_constant<int, 8> c8;
         constexpr int GT = decltype(gc)::value;
-        const int wn = pick_wn(N);
-        // one-wave workgroups of 32 rows for a single token block: four times the workgroups (304 at
-        // 9728 rows), each with a wave-private X ring
-        // Tiles measured on MI355X at 9728x2560 (512 / 128 tokens): 128 x 96 52.9 / 33.0 us,
-        // 128 x 64 57.9 / 27.7, 128 x 128 58.7 / 38.9; two or more row blocks per wave
-        // (256 x 96, 256 x 64, 128 x 96 over 2 waves, ...) 66-82 / 40-72; and staging W
-        // through LDS in 3-step chunks did not beat the loads straight into registers.
-        // (At 512 tokens, 128 x 160 tiles with 1 wave per SIMD, 256 x 128 tiles of 8 waves and
-        // W staged through LDS in 4-step chunks by 16-byte DMAs were no faster either.)
-        // Above 128 tokens: 256 x 96 tiles of 8 waves (one 32-row block each, W in registers)
-        // with a 3-step ring, 228 workgroups at 9728 x 512: 44.6-45.1 us per call against
-        // 46.3-47.2 for 128 x 96 tiles of 4 waves with a 4-step ring (a 4-step ring with 8 waves:
-        // 45.7-46.4; a 2-step ring: 60; the token tiles of a row tile on one XCD: no change).
-        // At 128 tokens the 4-step ring of 4 waves stays (3 steps: 26.2 us, 2: 41.1, 128 x 32
-        // tiles: 25.2, 256 x 32 tiles of 8 waves: 34.3, against 24.0).
-        const int st = wn == 1 ? static_cast<int>(kTooLarge)
-                       : wn == 2
-                           ? launch_direct<GT, 2, 4, 4>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream)
-                           : launch_direct<GT, 3, 3, 8>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
+        const int st = tl.kind == kTile128x32   ? go(gc, c1, c4, c4)
+                       : tl.kind == kTile128x64 ? go(gc, c2, c4, c4)
+                       : tl.kind == kTile256x96 ? go(gc, c3, c3, c8)
+                                                : static_cast<int>(kTooLarge);
         if (st != kTooLarge) return st;  // (rows whose tile passes the 32-bit offsets: the smallest tile)
-        return launch_direct<GT, 1, 4, 1>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, stream);
+        return launch_direct<GT, 1, 4, 1, kSplitNone>(w, xh, xinv, y, M, N, K, ikp, group_size, irb, sl, stream);
     };
     return group_size == 64 ? tiles(std::integral_constant<int, 64>{}) : tiles(std::integral_constant<int, 0>{});
 }
@@ -967,7 +1162,7 @@ int launch_i4_matmul_noalloc(const uint8_t *w, const float *x, float *y, int M, 
     if (mfma) {
         const int st = noalloc_scratch(&ws);
         if (st != kOk) return st;
-        return matmul_mfma(w, x, y, M, K, N, group_size, ws, stream);
+        return matmul_mfma(w, x, y, M, K, N, group_size, ws, tile_plan(M, K, N), nullptr, stream);
     }
     // One matvec per token column under a scratch set with no buffers: a kernel that would
     // need split-K slots is not chosen, and nothing is allocated.
@@ -991,11 +1186,22 @@ int launch_i4_matmul(const uint8_t *w, const float *x, float *y, int M, int K, i
         return launch_skinny(w, x, y, M, K, N, g, static_cast<float *>(part), slots, stream);
     }
     if (!mfma_applies(M, K, N, group_size)) return matmul_by_columns(w, x, y, M, K, N, group_size, stream);
-    void *ws = nullptr;
-    const int st = scratch_prefill(stream, prefill_scratch_bytes(K, N), &ws);  // the stream's (or scope's) buffer
-    if (st != kOk) return st;
-    const int mst = matmul_mfma(w, x, y, M, K, N, group_size, static_cast<unsigned char *>(ws), stream);
-    return mst == kTooLarge ? matmul_by_columns(w, x, y, M, K, N, group_size, stream) : mst;
+    const TilePlan tl = tile_plan(M, K, N);
+    void *ws = nullptr;  // the stream's (or scope's) buffer
+    unsigned long long *arrivals = nullptr;
+    if (tl.KS > 1 && (scratch_prefill(stream, part_offset(K, N) + tl.part_bytes, &ws) != kOk ||
+                      scratch_split_slots(stream, tl.tiles, &arrivals) != kOk)) {
+        // no room for the partials (a capture, or memory is short): the slices one after the other
+        ws = nullptr;
+        arrivals = nullptr;
+        (void)hipGetLastError();
+    }
+    if (!ws) {
+        const int st = scratch_prefill(stream, prefill_scratch_bytes(K, N), &ws);
+        if (st != kOk) return st;
+    }
+    const int st = matmul_mfma(w, x, y, M, K, N, group_size, static_cast<unsigned char *>(ws), tl, arrivals, stream);
+    return st == kTooLarge ? matmul_by_columns(w, x, y, M, K, N, group_size, stream) : st;
 }
 
 }  // namespace tqhip
