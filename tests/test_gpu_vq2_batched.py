@@ -54,3 +54,24 @@ def test_no_tokens_and_one_token(gpu):
     w, x = gpu.synth_vq2(40, 64, seed=5), gpu.synth_normal(64, seed=6)
     gpu.lib().tqhip_dispatch_matmul_vq2(w.ctypes.data, x.ctypes.data, None, 40, 64, 0)  # nothing to do
     assert np.array_equal(gpu.matmul_vq2(w, x, 40, 64, 1), gpu.matvec_vq2(w, x, 40, 64))
+
+
+# rows past 1024 elements, at least 256 per CU: the table taken slab by slab. Rows that are not a whole
+# number of slabs (1040, 2000 with an odd number of dwords), one to three batches a wave, more
+# workgroups than CUs (200003 rows), the shortest and a long row; and an infinite codebook entry 0,
+# which must not reach a row through the zero entries past its end.
+@pytest.mark.parametrize("M,K", [(65536, 1040), (65539, 2000), (70001, 1536), (151936, 1088), (200003, 1040),
+                                 (66000, 4112)])
+def test_long_row_table_matches_oracle(gpu, orc, M, K):
+    w, x = gpu.synth_vq2(M, K, seed=M + K), gpu.synth_normal(K, seed=K)
+    dx, dy = gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(4 * M)
+    for entry0 in (None, np.inf):
+        if entry0 is not None:
+            w[0:8] = np.frombuffer(np.full(4, entry0, np.float16).tobytes(), np.uint8)
+        want = orc.matvec_vq2(w, x, M, K, threads=16)
+        dw = gpu.DeviceBuffer.from_array(w)
+        gpu.lib().tqhip_memset(dy.ptr, 0xFF, 4 * M)  # every row must be written
+        gpu.matvec_vq2_dev(dw, dx, dy, M, K)
+        got, fin = dy.download(np.float32, M), np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), fin) and (entry0 is not None or fin.all())
+        assert rel_l2(got[fin], want[fin]) <= 1e-5

@@ -4,11 +4,13 @@
 // reference's matvec_vq2_ref (kernels/matvec/matvec_vq2_ref.cpp:52-81), on the
 // layout [codebook 256 x 4 fp16 = 2048 B][out_dim x in_dim/4 uint8 indices].
 //
-// Four kernels:
+// Five kernels:
 // - vq2_matvec_table (index rows 16-byte aligned, in_dim <= 1024, at least 256 rows per CU):
 //   per workgroup a table of every codebook entry's dot product with every 4-element block of
 //   x, built with fp32 MFMAs in LDS; a lookup is then one 4-byte LDS read and one add (see its
 //   comment).
+// - vq2_matvec_slabs (rows past 1024, index rows dword-aligned, at least 256 rows per CU): the same
+//   table for one slab of 512 elements after the other.
 // - vq2_matvec_copies (index rows dword-aligned, in_dim % 16 == 0): 16 bank-
 //   interleaved fp32 copies of the codebook in LDS make every lookup
 //   conflict-free; tiles of 4 rows per wave, the next tile's index dwords in
@@ -590,6 +592,35 @@ __device__ inline float tab_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
+// Per batch: the 4 row sums of each lane added over its 16 lanes by halving exchanges
+// (row_mirror, row_half_mirror, then quad swaps); lanes 4 m + 0 of each 16 keep row 4 m + rho's
+// total. y: the workgroup's rows.
+template <int BMAX>
+__device__ inline void tab_row_sums(const float (&acc)[BMAX][4], float *y, int nrows, int mynb, int wave, int lane) {
+    const int rho = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < BMAX; ++i) {
+        if (i < mynb) {
+            float v0 = acc[i][0], v1 = acc[i][1], v2 = acc[i][2], v3 = acc[i][3];
+            const bool u8 = lane & 8, u4 = lane & 4;
+            {
+                const float lo0 = v0 + tab_dpp<0x140>(v0), hi0 = v2 + tab_dpp<0x140>(v2);
+                const float lo1 = v1 + tab_dpp<0x140>(v1), hi1 = v3 + tab_dpp<0x140>(v3);
+                v0 = u8 ? hi0 : lo0;
+                v1 = u8 ? hi1 : lo1;
+            }
+            {
+                const float lo = v0 + tab_dpp<0x141>(v0), hi = v1 + tab_dpp<0x141>(v1);
+                v0 = u4 ? hi : lo;
+            }
+            v0 += tab_dpp<0x4E>(v0);
+            v0 += tab_dpp<0xB1>(v0);
+            const int row = kTabBatchRows * (wave + kTabWaves * i) + 4 * ((lane >> 2) & 3) + rho;
+            if ((lane & 3) == 0 && row < nrows) y[row] = v0;
+        }
+    }
+}
+
 template <int BMAX>
 __global__ __launch_bounds__(64 * kTabWaves) void vq2_matvec_table(const uint8_t *__restrict__ w,
                                                                    const float *__restrict__ x,
@@ -732,30 +763,169 @@ __global__ __launch_bounds__(64 * kTabWaves) void vq2_matvec_table(const uint8_t
         }
     }
 
-    // 4. per batch: the 4 row sums of each lane added over its 16 lanes by halving exchanges
-    //    (row_mirror, row_half_mirror, then quad swaps); lanes 4 m + 0 of each 16 keep row
-    //    4 m + rho's total
+    // 4. the row sums
+    tab_row_sums<BMAX>(acc, y + r0, nrows, mynb, wave, lane);
+}
+
+// ---- Dot-product table, rows past 1024 elements (large launches, index rows dword-aligned).
+// The table of vq2_matvec_table for rows that its two passes do not cover: a row is taken in slabs of
+// 128 index bytes (32 dwords d, 512 elements), each with a 128 KB table of two 64 KB sub-tables:
+//   slab s, sub-table h (d = 32 s + 2 q + h): entry (c, byte j, q) at byte
+//   h * 65536 + 256 c + 64 j + 4 q holds T[c][4 d + j], and 0 past the row end.
+// Lane (rho = lane / 16, q = lane % 16) loads 8 bytes, dwords 2 q and 2 q + 1 of the slab, of rows
+// 16 (wave + 16 i) + 4 r + rho (r = 0..3): a load instruction moves 4 x 128 contiguous bytes. A slab's
+// index dwords sit in one of two register sets, requested while the slab before is looked up.
+// Table, lookups and bank layout as in vq2_matvec_table; the same fp32 products and additions.
+// Measured on MI355X (cold weights) against vq2_matvec_copies, which reads 16 LDS bytes and does four
+// FMAs a lookup: 151936x2560 43.8 -> 32.0, 151936x1536 29.0 -> 20.2, 65536x2560 20.1 -> 16.0,
+// 100000x2000 22.5 -> 19.3, 66000x4096 28.8 -> 27.5 us. Bound by the table and lookup phases (~6 us a slab at 594 rows), not by the
+// index stream. Forming the next sub-table's tiles behind the current one's lookups (one barrier per
+// sub-table, 16 or 8 waves) was slower: 35-42 us at 151936x2560.
+constexpr int kSlabDwords = 32;     // index dwords of a slab
+constexpr int kSlabMaxDim = 1 << 20;
+constexpr int kSlabMaxBatches = 3;  // batches per wave (128 VGPRs): <= 768 rows per workgroup
+
+template <int BMAX>
+__global__ __launch_bounds__(64 * kTabWaves) void vq2_matvec_slabs(const uint8_t *__restrict__ w,
+                                                                   const float *__restrict__ x,
+                                                                   float *__restrict__ y, int M, int K,
+                                                                   int rows_per_wg) {
+    __shared__ __align__(16) unsigned char tab[2 * 65536];
+    typedef float f16v __attribute__((ext_vector_type(16)));
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = K / kVq2Dim, nd = nb / 4;  // index bytes and dwords per row
+    const int slabs = (nd + kSlabDwords - 1) / kSlabDwords;
+    const int r0 = blockIdx.x * rows_per_wg;
+    const int nrows = min(rows_per_wg, M - r0);
+    if (nrows <= 0) return;
+    const uint16_t *cbh = reinterpret_cast<const uint16_t *>(w);
+    const int rho = lane >> 4, q = lane & 15;
+    const int nbatch = (nrows + kTabBatchRows - 1) / kTabBatchRows;
+    const int mynb = wave < nbatch ? (nbatch - 1 - wave) / kTabWaves + 1 : 0;  // this wave's batches (<= BMAX)
+
+    // 1. table operands, raw: tile t = 2 wave + tt covers entries 32 (t & 7) + 0..31 and, with ts =
+    //    t / 8, positions of sub-table ts / 2, bytes 2 (ts & 1) + 0..1; MFMA column n = lane % 32 is
+    //    byte j = 2 (ts & 1) + n / 16 of dword 32 s + 2 (n % 16) + ts / 2. (ts is the same for tt = 0, 1.)
+    const int ts = wave >> 2, j = 2 * (ts & 1) + ((lane >> 4) & 1);
+    const int pos0 = 4 * (2 * (lane & 15) + (ts >> 1)) + j;  // the column's index byte within a slab
+    uint16_t cbr[2][2];
+    float xr[2];
+    auto load_x = [&](int s) {
+        const int b = 4 * kSlabDwords * s + pos0;
 #pragma unroll
-    for (int i = 0; i < BMAX; ++i) {
-        if (i < mynb) {
-            float v0 = acc[i][0], v1 = acc[i][1], v2 = acc[i][2], v3 = acc[i][3];
-            const bool u8 = lane & 8, u4 = lane & 4;
-            {
-                const float lo0 = v0 + tab_dpp<0x140>(v0), hi0 = v2 + tab_dpp<0x140>(v2);
-                const float lo1 = v1 + tab_dpp<0x140>(v1), hi1 = v3 + tab_dpp<0x140>(v3);
-                v0 = u8 ? hi0 : lo0;
-                v1 = u8 ? hi1 : lo1;
-            }
-            {
-                const float lo = v0 + tab_dpp<0x141>(v0), hi = v1 + tab_dpp<0x141>(v1);
-                v0 = u4 ? hi : lo;
-            }
-            v0 += tab_dpp<0x4E>(v0);
-            v0 += tab_dpp<0xB1>(v0);
-            const int row = kTabBatchRows * (wave + kTabWaves * i) + 4 * ((lane >> 2) & 3) + rho;
-            if ((lane & 3) == 0 && row < nrows) y[r0 + row] = v0;
-        }
+        for (int k2 = 0; k2 < 2; ++k2) xr[k2] = x[b < nb ? kVq2Dim * b + 2 * k2 + (lane >> 5) : 0];
+    };
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+            cbr[tt][k2] = cbh[kVq2Dim * (32 * ((2 * wave + tt) & 7) + (lane & 31)) + 2 * k2 + (lane >> 5)];
+    load_x(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+
+    // 2. the index loads of this wave's first batch (out-of-range offsets read 0 and fetch nothing;
+    //    an odd last dword's pair ends in the next row, whose bytes meet zero entries)
+    const uint8_t *idx = w + kVq2CodebookBytes + static_cast<size_t>(r0) * nb;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(idx), static_cast<short>(0),
+                                                                        nrows * nb, kBufferFlags);
+    uint2 qd[2][BMAX][4];
+    auto issue = [&](uint2 (&d)[4], int i, int s) {
+        const int row0 = kTabBatchRows * (wave + kTabWaves * i) + rho, dw = kSlabDwords * s + 2 * q;
+        const bool ok = i < mynb && dw < nd;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            d[r] = __builtin_bit_cast(
+                uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, ok ? (row0 + 4 * r) * nb + 4 * dw : 0xFFFFFFF0u, 0, 0));
+    };
+    issue(qd[0][0], 0, 0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+
+    float av[2][2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2) av[tt][k2] = half_bits(cbr[tt][k2]);
+    unsigned loff[2][4], sel[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const unsigned jl = (k + rho) & 3;
+        loff[0][k] = 64u * jl + 4u * q;
+        loff[1][k] = loff[0][k] | 0x10000u;
+        sel[k] = 0x0C020000u | ((4u + jl) << 8);  // bytes: loff.0, index byte jl, loff.2, zero
     }
+    auto build = [&](int s) {
+        const bool pad = 4 * kSlabDwords * s + pos0 >= nb;  // the column lies past the row end: zero entries
+        const float b0 = pad ? 0.f : xr[0], b1 = pad ? 0.f : xr[1];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const int c0 = 32 * ((2 * wave + tt) & 7);
+            f16v d = {};
+            d = __builtin_amdgcn_mfma_f32_32x32x2f32(av[tt][0], b0, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_32x32x2f32(av[tt][1], b1, d, 0, 0, 0);
+            const unsigned base = ((ts >> 1) << 16) + 64 * j + 4 * (lane & 15);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {  // D row 8 (r / 4) + 4 (lane / 32) + r % 4 = entry offset
+                const int c = c0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                *reinterpret_cast<float *>(tab + base + 256 * c) = pad ? 0.f : d[r];
+            }
+        }
+    };
+
+    float acc[BMAX][4];
+#pragma unroll
+    for (int i = 0; i < BMAX; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][r] = 0.f;
+    // 3. the first table, then the rest of the first two slabs' index stream
+    build(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 1; i < BMAX; ++i) issue(qd[0][i], i, 0);
+#pragma unroll
+    for (int i = 0; i < BMAX; ++i) issue(qd[1][i], i, 1);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    // 4. a slab's lookups, then the next slab's table and the loads of the one after it into the
+    //    registers that the lookups have freed
+    auto slab = [&](uint2 (&d)[BMAX][4], int s) {
+        if (s + 1 < slabs) load_x(s + 1);
+#pragma unroll
+        for (int i = 0; i < BMAX; ++i) {
+            if (i < mynb) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float a = 0.f;  // (a slab's sum from zero: shorter chains of roundings)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const unsigned dw = h ? d[i][r].y : d[i][r].x;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            a += *reinterpret_cast<const float *>(tab + __builtin_amdgcn_perm(dw, loff[h][k], sel[k]));
+                    }
+                    acc[i][r] += a;
+                }
+            }
+        }
+        if (s + 1 >= slabs) return;
+        if (s + 2 < slabs) {
+#pragma unroll
+            for (int i = 0; i < BMAX; ++i) issue(d[i], i, s + 2);
+        }
+        __syncthreads();  // every lookup of this slab is done
+        build(s + 1);
+        __syncthreads();
+    };
+    for (int s = 0; s < slabs; s += 2) {
+        slab(qd[0], s);
+        if (s + 1 < slabs) slab(qd[1], s + 1);
+    }
+
+    tab_row_sums<BMAX>(acc, y + r0, nrows, mynb, wave, lane);
 }
 
 }  // namespace
@@ -785,6 +955,18 @@ int launch_vq2_matvec(const uint8_t *w, const float *x, float *y, int out_dim, i
             case 4: hipLaunchKernelGGL(vq2_matvec_table<4>, dim3(grid), dim3(64 * kTabWaves), 0, stream, w, x, y, out_dim, in_dim, rpw); break;
             default: return kBadShape;  // unreachable: rpw <= kMaxRows
         }
+        return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
+    }
+    if (aligned && in_dim > kTabMaxDim && in_dim <= kSlabMaxDim &&
+        static_cast<long long>(out_dim) >= static_cast<long long>(kTabMinRowsPerCu) * cus) {
+        // longer rows, as many: the table slab by slab (below 256 rows per CU its tables cost what
+        // the lookups save: 32768x2560 12.2 against 12.0 us)
+        constexpr int kMaxRows = kTabWaves * kTabBatchRows * kSlabMaxBatches;
+        const int grid = cus * ((out_dim - 1) / (cus * kMaxRows) + 1);
+        const int rpw = (out_dim + grid - 1) / grid;
+        const int batches = ((rpw + kTabBatchRows - 1) / kTabBatchRows + kTabWaves - 1) / kTabWaves;
+        const auto kernel = batches == 1 ? vq2_matvec_slabs<1> : batches == 2 ? vq2_matvec_slabs<2> : vq2_matvec_slabs<3>;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kTabWaves), 0, stream, w, x, y, out_dim, in_dim, rpw);
         return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
     }
     if (aligned) {
