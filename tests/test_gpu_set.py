@@ -209,3 +209,73 @@ def test_non_finite_activation_stays_in_its_matrix(gpu, orc):
             assert not np.any(np.isfinite(g)), f"{name}: finite outputs from a NaN activation"
         else:
             assert np.array_equal(g, c), f"{name}: changed by another matrix's NaN activation"
+
+
+SET_SHAPES = [(1, 4), (17, 32), (33, 96), (65, 860), (2048, 1024), (2049, 1028), (31, 2080), (129, 4864), (16, 8224),
+              (2050, 10240), (7, 10244)]  # (10244: past the set kernel's rows)
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+@pytest.mark.parametrize("M,K", SET_SHAPES)
+def test_group_sizes_at_the_edges(gpu, orc, G, M, K):
+    """The set kernel's group sizes at the edges of its shapes (row halves, slots, rows that end inside
+    a weight group or a block of 64 activations), alone and in a set with a second matrix. Each row
+    is held to its rounding: x to 2^-23 of the largest |x| of its 64 (groups of 128 past the set kernel: 2^-22
+    of the largest of 128), then at most 16 roundings (the half-group's value, the slots and the wave sum)
+    of its terms, each at most scale * 30 * |x|. Half of the activations are ties of that rounding."""
+    rng = np.random.default_rng(K * 7 + M + G)
+    x = rng.standard_normal(K).astype(np.float32)
+    x[::2] = (np.sign(x[::2]) * (np.floor(np.abs(x[::2]) * 2**18) + 0.5) * 2.0**-18).astype(np.float32)
+    w = gpu.synth_i4(M, K, G, seed=5)
+    w2 = gpu.synth_i4(24, K, G, seed=6)
+    got = []
+    for mats in ([(w, M)], [(w2, 24), (w, M)]):
+        dev = [(gpu.DeviceBuffer.from_array(b), gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(4 * m), m, K)
+               for b, m in mats]
+        if len(mats) == 1:
+            gpu.matvec_i4_dev(dev[0][0], dev[0][1], dev[0][2], M, K, G)
+        else:
+            gpu.matvec_i4_set_dev(gpu.i4_set(dev), G)
+        gpu.synchronize()
+        got.append(dev[-1][2].download(np.float32, M))
+    wd = orc.dequant_i4_matrix_f64(w, M, K, G)
+    want = wd @ x.astype(np.float64)
+    groups = -(-K // G)
+    scale = w.reshape(M, groups, 4 + G // 2)[:, :, :2].copy().view(np.float16)[:, :, 0].astype(np.float64)
+    scale = np.repeat(np.abs(scale), G, axis=1)[:, :K]
+    block = 64 if K <= 10240 else max(G, 64)
+    peak = np.repeat([np.abs(x[b:b + block]).max() for b in range(0, K, block)], block)[:K].astype(np.float64)
+    step = 2.0**-23 if K <= 10240 else 2.0**-22
+    bound = step * (np.abs(wd) @ peak) + 16 * 2.0**-24 * 30 * (scale @ np.abs(x.astype(np.float64)))
+    for y, what in zip(got, ("alone", "in a set")):
+        err = np.abs(y - want)
+        assert np.all(err <= bound), f"{what}: worst row err/bound = {float(np.max(err / bound)):.3f}"
+    if K <= 10240:
+        assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+def test_extreme_activations_by_group_size(gpu, orc, G):
+    """Activations whose scaled value is the largest that 24 bits hold, the largest and the smallest
+    floats: products of the ends of the range against the oracle, and an infinity or a NaN in every
+    row that reads it."""
+    M, K = 48, 1344
+    w = gpu.synth_i4(M, K, G, seed=9)
+    wd = orc.dequant_i4_matrix_f64(w, M, K, G)
+    dw, dy = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer(4 * M)
+    base = np.random.default_rng(1).standard_normal(K).astype(np.float32)
+    for peak in (np.float32(1) - np.float32(2.0**-24), np.float32(3e36), np.float32(1e-38), np.float32(2.0**-149)):
+        x = (base / np.abs(base).max() * peak).astype(np.float32)
+        x[::7] = peak
+        gpu.matvec_i4_dev(dw, gpu.DeviceBuffer.from_array(x), dy, M, K, G)
+        gpu.synchronize()
+        want = wd @ x.astype(np.float64)
+        # 1e-6 of the row's terms; a result below the normal floats is held to a few of their last units
+        bound = 1e-6 * (np.abs(wd) @ np.abs(x.astype(np.float64))) + 64 * 2.0**-149
+        assert np.all(np.abs(dy.download(np.float32, M) - want) <= bound), peak
+    for bad in (np.inf, np.nan):
+        x = base.copy()
+        x[K - 1] = bad
+        gpu.matvec_i4_dev(dw, gpu.DeviceBuffer.from_array(x), dy, M, K, G)
+        gpu.synchronize()
+        assert not np.isfinite(dy.download(np.float32, M)).any()

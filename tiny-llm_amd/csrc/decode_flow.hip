@@ -270,7 +270,7 @@ __device__ __attribute__((always_inline)) bool flow_rows(const RowsJob &j, const
         const float2 h = hs[ru];
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
-            const float v = half_group_int(cd[r * NS + sl], hd[r * NS + sl], xv, h);
+            const float v = half_group_int<3>(cd[r * NS + sl], hd[r * NS + sl], xv, h);
             if (unit < U) p[r] += v;
         }
     }

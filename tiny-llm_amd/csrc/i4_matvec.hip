@@ -1552,6 +1552,11 @@ int launch_i4_matvec(const uint8_t *w, const float *x, float *y, int out_dim, in
     if (!w || !x || !y) return kBadShape;  // nothing is launched on a null operand
     const size_t rb = i4_row_bytes(in_dim, group_size);
     const bool fast_group = (group_size % 8 == 0) && group_size >= 40;
+    if (group_size == 32) {
+        const I4Mat m{w, x, y, out_dim, in_dim};
+        const int st = launch_i4_matvec_set_fit(1, &m, group_size, stream);
+        if (st != kNotFused) return st;
+    }
     if (!fast_group || rb * kTile * 2 >= (1ull << 31))
         return launch_i4_matvec_generic(w, x, y, out_dim, in_dim, group_size, stream);
     Geom gm = one_matrix_geom(w, y, out_dim, in_dim, group_size);

@@ -1,5 +1,5 @@
-// i4_set.hip -- one launch over a set of i4 HQQ@64 matvecs, each with its own
-// activation vector, output, row count and row length.
+// i4_set.hip -- one launch over a set of i4 HQQ matvecs of one group size (32, 64 or 128), each
+// with its own activation vector, output, row count and row length.
 //
 // A decoder layer's matvec set (q, k, v, o, gate, up, down: four distinct
 // activation vectors) is about 8 MB at Qwen2.5-0.5B scale, a microsecond or two
@@ -22,9 +22,13 @@
 //     activation digits, exact before a per-half-group fp32 epilogue.
 // The same kernel serves single-matrix and pair / qkv launches of decode size
 // (launch_i4_matvec_set_fit), so a matrix gives the same bits alone or in a set.
-// Numerics: the only rounding before the epilogue is x -> X (relative 2^-23 of the
-// group's largest |x|); measured rel L2 ~4e-7 against the double-accumulating reference
-// (kernels/matvec/matvec_i4_ref.cpp:45-103).
+// Numerics: the only rounding before the epilogue is x -> X (at most 2^-23 of the largest |x| of
+// 64, groups of 32: 2^-25); measured rel L2 1.4e-7 to 1.8e-7 (groups of 32: 1.0e-7) against the
+// double-accumulating reference (kernels/matvec/matvec_i4_ref.cpp:45-103).
+// Groups of 32 and 128 took a wave-per-row FMA kernel and the split-K and register-path MFMA
+// kernels before; measured cold, us: 128: 896x4864 8.0 -> 5.0, 2560x4096 8.1 -> 4.4, 9728x2560
+// 8.4 -> 7.4, 2560x9728 12.5 -> 7.1; 32: 4864x896 13.5 -> 4.2, 9728x2560 63 -> 9.4, 151936x2560
+// 899 -> 68.
 #include "i4_set_core.h"
 
 #include <algorithm>
@@ -51,11 +55,16 @@ struct SetArgs {
     SetPrologue pro;  // XM != 0 instances only
 };
 
+// Digits of the activations by weight group size; see stage_x.
+constexpr int set_digits(int G) { return G == 32 ? 4 : 3; }
+
 // XM: the activation prologue (0 none; 1 x = silu(x) * x2; 2 x = rmsnorm((x + d1) + d2) * nw,
 // workgroup 0 storing the sum to hout), with its operands in pro. GLU: every row of m is computed
 // together with the same row of w2 (a matrix of m's shape reading the same x), and the row's
 // output is swiglu(m row, w2 row), as the separate outputs would give it in a SwiGLU prologue.
-template <int S, int R, int XM, bool GLU = false>
+// G: the weights' group size. The activations' exponents are per 64 elements whatever G is, and a
+// lane's half-group of 32 elements lies in one weight group, so G only moves the addresses.
+template <int S, int R, int XM, bool GLU = false, int G = 64>
 __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char *lds, const SetPrologue &pro,
                                          const uint8_t *w2 = nullptr) {
     // 16-byte activation loads per thread: the chunks of the widest row of this shape
@@ -65,10 +74,15 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int U = 2 * ((m.K + 63) / 64), rb = 18 * U;  // half-groups and bytes per row
+    constexpr int kHalves = G / 32, kGroupBytes = kI4Header + G / 2;  // half-groups and bytes of a group
+    const int U = 2 * ((m.K + 63) / 64);                              // half-groups of activations per row
+    const int rb = G == 64 ? 18 * U : (m.K + G - 1) / G * kGroupBytes;  // bytes per row
+    // half-groups that are summed (G = 64: all of U are in the row; else the last one may lie past it)
+    const int UW = G == 64 ? U : (m.K + 31) / 32;
+    constexpr int P = set_digits(G);
     const int C = 8 * U;                                 // 16-byte activation chunks the rows read
     unsigned char *xp = lds;                                              // C / 2 blocks of operands
-    float2 *hs = reinterpret_cast<float2 *>(lds + (C / 2) * kBlockBytes);  // U (sum(X), 2^-f)
+    float2 *hs = reinterpret_cast<float2 *>(lds + (C / 2) * block_bytes(P));  // U (sum(X), 2^-f)
 
     // 1. the activations first: chunk t + kSetThreads i, clamped to the last one (zeroed past K
     // in stage_x). (Plain 16-byte loads: with a 16-byte buffer load whose elements are used
@@ -118,10 +132,10 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
         const int r = q / NS, sl = q % NS;
         const int rr = GLU ? r % R : r;  // GLU: rows R.. are the same rows of w2
         const int unit = u + 64 * sl;
-        const int off = (S == 0 ? 2 * rr + half : rr) * rb + (kI4Header + 32) * (unit >> 1);
+        const int off = (S == 0 ? 2 * rr + half : rr) * rb + kGroupBytes * (unit / kHalves);
         const __amdgpu_buffer_rsrc_t rs = GLU && r >= R ? wr2 : wr;
         hd[q] = __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
-        cd[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + kI4Header + 16 * (unit & 1), 0, 0);
+        cd[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + kI4Header + 16 * (unit % kHalves), 0, 0);
     };
 #pragma unroll
     for (int q = 0; q < NFIRST; ++q) issue(q);
@@ -157,7 +171,7 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
         for (int i = 0; i < NX; ++i) xq[i] = rms_apply(xq[i], scale, pw[i]);
     }
 #pragma unroll
-    for (int i = 0; i < NX; ++i) stage_x(xq[i], t + kSetThreads * i, Kc, C, xp, hs);
+    for (int i = 0; i < NX; ++i) stage_x<P>(xq[i], t + kSetThreads * i, Kc, C, xp, hs);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = NFIRST; q < NU; ++q) issue(q);
@@ -172,10 +186,10 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
     for (int sl = 0; sl < NS; ++sl) {
         const int unit = u + 64 * sl;
         const int ru = min(unit, U - 1);
-        unsigned xv[24];
-        const v4i *src = reinterpret_cast<const v4i *>(xp + ru * 4 * kBlockBytes);
+        unsigned xv[8 * P];
+        const v4i *src = reinterpret_cast<const v4i *>(xp + ru * 4 * block_bytes(P));
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
+        for (int k = 0; k < 2 * P; ++k) {
             const v4i v = src[k];
             xv[4 * k] = v[0];
             xv[4 * k + 1] = v[1];
@@ -185,8 +199,8 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
         const float2 h = hs[ru];
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
-            const float v = half_group_int(cd[r * NS + sl], hd[r * NS + sl], xv, h);
-            if (unit < U) p[r] += v;
+            const float v = half_group_int<P>(cd[r * NS + sl], hd[r * NS + sl], xv, h);
+            if (unit < UW) p[r] += v;
         }
     }
 #pragma unroll
@@ -205,7 +219,7 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
 // SMAX: the largest shape in the launch (the register budget follows it); R: rows per
 // half-wave for the short rows; RL: rows per wave for the long rows (two rows share the
 // activation operands each wave reads from LDS and halve the workgroups that convert x).
-template <int SMAX, int R, int RL, int XM, int C>
+template <int SMAX, int R, int RL, int XM, int C, int G = 64>
 __global__ __launch_bounds__(kSetThreads) void i4_matvec_set(SetArgs<C> a) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int b = blockIdx.x;
@@ -218,17 +232,17 @@ __global__ __launch_bounds__(kSetThreads) void i4_matvec_set(SetArgs<C> a) {
         if (i == j) m = a.m[i];
     const int blk = b - m.blk0;
     if (m.shape == 0) {
-        set_rows<0, R, XM>(m, blk, lds, a.pro);
+        set_rows<0, R, XM, false, G>(m, blk, lds, a.pro);
     } else if (SMAX <= 1 || m.shape == 1) {
-        set_rows<1, RL, XM>(m, blk, lds, a.pro);
+        set_rows<1, RL, XM, false, G>(m, blk, lds, a.pro);
     } else if (SMAX <= 2 || m.shape == 2) {
-        set_rows<2, RL, XM>(m, blk, lds, a.pro);
+        set_rows<2, RL, XM, false, G>(m, blk, lds, a.pro);
     } else if (SMAX <= 3 || m.shape == 3) {
-        set_rows<3, RL, XM>(m, blk, lds, a.pro);
+        set_rows<3, RL, XM, false, G>(m, blk, lds, a.pro);
     } else if (SMAX <= 4 || m.shape == 4) {
-        set_rows<4, RL, XM>(m, blk, lds, a.pro);
+        set_rows<4, RL, XM, false, G>(m, blk, lds, a.pro);
     } else {
-        set_rows<5, RL, XM>(m, blk, lds, a.pro);
+        set_rows<5, RL, XM, false, G>(m, blk, lds, a.pro);
     }
 }
 
@@ -244,35 +258,35 @@ __global__ __launch_bounds__(kSetThreads) void i4_matvec_glu(SetArgs<2> a) {
 }
 
 // Shape of a matrix in the set kernel, or -1 when the kernel does not take it:
-// G = 64, K % 4 == 0 and x 16-byte aligned (whole 16-byte activation loads), K <= 10240.
+// G = 32, 64 or 128, K % 4 == 0 and x 16-byte aligned (whole 16-byte activation loads), K <= 10240.
 int set_shape(const I4Mat &mt, int group_size) {
-    if (group_size != 64 || mt.K % 4 != 0 || mt.K > kSetMaxSlots * 64 * 32 ||
+    if ((group_size != 64 && group_size != 32 && group_size != 128) || mt.K % 4 != 0 || mt.K > kSetMaxSlots * 64 * 32 ||
         (reinterpret_cast<uintptr_t>(mt.x) & 15) != 0)
         return -1;
     return mt.K <= 1024 ? 0 : (mt.K + 64 * 32 - 1) / (64 * 32);
 }
 
-template <int R, int RL, int XM, int C>
+template <int R, int RL, int XM, int C, int G = 64>
 void launch_r(int smax, const dim3 &grid, const dim3 &block, size_t lds, hipStream_t stream, const SetArgs<C> &a) {
     switch (smax) {
-        case 0: hipLaunchKernelGGL((i4_matvec_set<0, R, 1, XM, C>), grid, block, lds, stream, a); break;
-        case 1: hipLaunchKernelGGL((i4_matvec_set<1, R, RL, XM, C>), grid, block, lds, stream, a); break;
-        case 2: hipLaunchKernelGGL((i4_matvec_set<2, R, RL, XM, C>), grid, block, lds, stream, a); break;
-        case 3: hipLaunchKernelGGL((i4_matvec_set<3, R, RL, XM, C>), grid, block, lds, stream, a); break;
-        case 4: hipLaunchKernelGGL((i4_matvec_set<4, R, RL, XM, C>), grid, block, lds, stream, a); break;
-        default: hipLaunchKernelGGL((i4_matvec_set<5, R, RL, XM, C>), grid, block, lds, stream, a); break;
+        case 0: hipLaunchKernelGGL((i4_matvec_set<0, R, 1, XM, C, G>), grid, block, lds, stream, a); break;
+        case 1: hipLaunchKernelGGL((i4_matvec_set<1, R, RL, XM, C, G>), grid, block, lds, stream, a); break;
+        case 2: hipLaunchKernelGGL((i4_matvec_set<2, R, RL, XM, C, G>), grid, block, lds, stream, a); break;
+        case 3: hipLaunchKernelGGL((i4_matvec_set<3, R, RL, XM, C, G>), grid, block, lds, stream, a); break;
+        case 4: hipLaunchKernelGGL((i4_matvec_set<4, R, RL, XM, C, G>), grid, block, lds, stream, a); break;
+        default: hipLaunchKernelGGL((i4_matvec_set<5, R, RL, XM, C, G>), grid, block, lds, stream, a); break;
     }
 }
 
-template <int XM, int C>
+template <int XM, int C, int G = 64>
 void launch_rr(int R, int RL, int smax, const dim3 &grid, const dim3 &block, size_t lds, hipStream_t stream,
                const SetArgs<C> &a) {
     if (R == 2)
-        RL == 2 ? launch_r<2, 2, XM, C>(smax, grid, block, lds, stream, a)
-                : launch_r<2, 1, XM, C>(smax, grid, block, lds, stream, a);
+        RL == 2 ? launch_r<2, 2, XM, C, G>(smax, grid, block, lds, stream, a)
+                : launch_r<2, 1, XM, C, G>(smax, grid, block, lds, stream, a);
     else
-        RL == 2 ? launch_r<1, 2, XM, C>(smax, grid, block, lds, stream, a)
-                : launch_r<1, 1, XM, C>(smax, grid, block, lds, stream, a);
+        RL == 2 ? launch_r<1, 2, XM, C, G>(smax, grid, block, lds, stream, a)
+                : launch_r<1, 1, XM, C, G>(smax, grid, block, lds, stream, a);
 }
 
 // Two long rows per wave when every long-row matrix of the launch has at least this many rows.
@@ -290,7 +304,8 @@ int long_rows_per_wave(const I4Mat *mats, const int *shape, int n) {
     return any ? 2 : 1;
 }
 
-int launch_set(const I4Mat *mats, const int *shape, int n, hipStream_t stream, const SetPrologue *pro = nullptr) {
+int launch_set(const I4Mat *mats, const int *shape, int n, int group_size, hipStream_t stream,
+               const SetPrologue *pro = nullptr) {
     SetArgs<kSetMaxMats> a{};
     if (pro) a.pro = *pro;
     int order[kSetMaxMats];
@@ -316,9 +331,23 @@ int launch_set(const I4Mat *mats, const int *shape, int n, hipStream_t stream, c
     }
     for (int k = n; k < kSetMaxMats; ++k) a.m[k] = a.m[n - 1];  // never selected (k >= n)
     a.n = n;
-    const size_t lds = static_cast<size_t>(umax) * (4 * kBlockBytes + 8);  // the widest row's operands
+    const size_t lds = static_cast<size_t>(umax) * (4 * block_bytes(set_digits(group_size)) + 8);  // the widest row's operands
     const dim3 grid(blocks), block(kSetThreads);
     const int xm = pro ? pro->kind : 0;
+    if (group_size != 64) {  // (prologue launches are G = 64 only)
+        if (xm) return kNotFused;
+        if (n <= kSetSmallMats) {
+            SetArgs<kSetSmallMats> s3{};
+            for (int k = 0; k < kSetSmallMats; ++k) s3.m[k] = a.m[k];
+            s3.n = a.n;
+            group_size == 32 ? launch_rr<0, kSetSmallMats, 32>(R, RL, smax, grid, block, lds, stream, s3)
+                             : launch_rr<0, kSetSmallMats, 128>(R, RL, smax, grid, block, lds, stream, s3);
+        } else {
+            group_size == 32 ? launch_rr<0, kSetMaxMats, 32>(R, RL, smax, grid, block, lds, stream, a)
+                             : launch_rr<0, kSetMaxMats, 128>(R, RL, smax, grid, block, lds, stream, a);
+        }
+        return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
+    }
     if (n <= kSetSmallMats) {  // the prologue launches always (launch_i4_matvec_set_pro)
         SetArgs<kSetSmallMats> s3{};
         for (int k = 0; k < kSetSmallMats; ++k) s3.m[k] = a.m[k];
@@ -343,6 +372,10 @@ int launch_set(const I4Mat *mats, const int *shape, int n, hipStream_t stream, c
 // 151936x896 (4748 workgroups) both take 19 us and at 151936x2560 the DMA ring wins
 // (39 vs 69 us).
 constexpr int kSetMaxBlocksPerCu = 8;
+// Groups of 128 have a faster kernel on the other side of the line: 19456x2560 (1216 workgroups)
+// 9.5 us here against 10.2, 32000x2560 (2000) 13.7 against 12.9. Groups of 32 have none: the FMA kernel takes
+// 335 us at 151936x896 against 22.6, and 899 at 151936x2560 against 68.
+constexpr int kSetMaxBlocksPerCu128 = 6;
 
 }  // namespace
 
@@ -360,7 +393,8 @@ bool set_fit_shapes(int n, const I4Mat *mats, int group_size, int *shape) {
     for (int i = 0; i < n; ++i)
         blocks += shape[i] == 0 ? (mats[i].M + 4 * kSetWaves - 1) / (4 * kSetWaves)
                                 : (mats[i].M + RL * kSetWaves - 1) / (RL * kSetWaves);
-    return blocks <= static_cast<long>(kSetMaxBlocksPerCu) * device_cu_count();
+    const int per_cu = group_size == 128 ? kSetMaxBlocksPerCu128 : kSetMaxBlocksPerCu;
+    return group_size == 32 || blocks <= static_cast<long>(per_cu) * device_cu_count();
 }
 
 }  // namespace
@@ -368,7 +402,7 @@ bool set_fit_shapes(int n, const I4Mat *mats, int group_size, int *shape) {
 int launch_i4_matvec_set_fit(int n, const I4Mat *mats, int group_size, hipStream_t stream) {
     int shape[kSetMaxMats];
     if (!set_fit_shapes(n, mats, group_size, shape)) return kNotFused;
-    return launch_set(mats, shape, n, stream);
+    return launch_set(mats, shape, n, group_size, stream);
 }
 
 bool i4_set_fit_takes(int n, const I4Mat *mats, int group_size) {
@@ -378,11 +412,11 @@ bool i4_set_fit_takes(int n, const I4Mat *mats, int group_size) {
 
 bool set_kernel_takes(int K, int group_size) {
     const I4Mat probe{nullptr, nullptr, nullptr, 1, K};  // (a null x is 16-byte aligned)
-    return K >= 1 && set_shape(probe, group_size) >= 0;
+    return K >= 1 && group_size == 64 && set_shape(probe, group_size) >= 0;
 }
 
 int launch_i4_matvec_set_pro(int n, const I4Mat *mats, int group_size, const SetPrologue &pro, hipStream_t stream) {
-    if (n < 1 || n > kSetSmallMats || pro.kind < 1 || pro.kind > 2) return kNotFused;
+    if (n < 1 || n > kSetSmallMats || pro.kind < 1 || pro.kind > 2 || group_size != 64) return kNotFused;
     const auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     if (!al(pro.x2) || !al(pro.d1) || !al(pro.d2) || !al(pro.nw) || !al(pro.hout) ||
         (pro.kind == 1 && !pro.x2) || (pro.kind == 2 && !pro.nw))
@@ -392,14 +426,14 @@ int launch_i4_matvec_set_pro(int n, const I4Mat *mats, int group_size, const Set
         shape[i] = set_shape(mats[i], group_size);
         if (shape[i] < 0 || mats[i].M < 1 || mats[i].x != mats[0].x || mats[i].K != mats[0].K) return kNotFused;
     }
-    return launch_set(mats, shape, n, stream, &pro);
+    return launch_set(mats, shape, n, group_size, stream, &pro);
 }
 
 int launch_i4_matvec_glu(const I4Mat &gate, const I4Mat &up, int group_size, const SetPrologue &pro,
                          hipStream_t stream) {
     const auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const int shape = set_shape(gate, group_size);
-    if (shape < 0 || set_shape(up, group_size) != shape || gate.M < 1 || up.M != gate.M || up.K != gate.K ||
+    if (group_size != 64 || shape < 0 || set_shape(up, group_size) != shape || gate.M < 1 || up.M != gate.M || up.K != gate.K ||
         up.x != gate.x || !gate.w || !up.w || !gate.x || !gate.y || pro.kind != 2 || !pro.nw || !al(pro.d1) ||
         !al(pro.d2) || !al(pro.nw) || !al(pro.hout))
         return kNotFused;
@@ -432,7 +466,8 @@ int launch_i4_matvec_set(int n, const I4Mat *mats, int group_size, hipStream_t s
     int shape[kSetMaxMats], nb = 0;
     for (int i = 0; i < n; ++i) {
         const int s = set_shape(mats[i], group_size);
-        if (s < 0) {
+        // (128: a matrix too large for the set kernel alone keeps its own kernel in a set, too)
+        if (s < 0 || (group_size == 128 && !i4_set_fit_takes(1, mats + i, group_size))) {
             const int st = launch_i4_matvec(mats[i].w, mats[i].x, mats[i].y, mats[i].M, mats[i].K, group_size, stream);
             if (st != kOk) return st;
             continue;
@@ -440,12 +475,12 @@ int launch_i4_matvec_set(int n, const I4Mat *mats, int group_size, hipStream_t s
         batch[nb] = mats[i];
         shape[nb++] = s;
         if (nb == kSetMaxMats) {
-            const int st = launch_set(batch, shape, nb, stream);
+            const int st = launch_set(batch, shape, nb, group_size, stream);
             if (st != kOk) return st;
             nb = 0;
         }
     }
-    return nb > 0 ? launch_set(batch, shape, nb, stream) : kOk;
+    return nb > 0 ? launch_set(batch, shape, nb, group_size, stream) : kOk;
 }
 
 }  // namespace tqhip

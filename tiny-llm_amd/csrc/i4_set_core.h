@@ -18,34 +18,55 @@ constexpr int kSetThreads = 64 * kSetWaves;
 constexpr int kSetMaxSlots = 5;   // wave-per-row slots of 64 half-groups: K <= 5 * 64 * 32
 
 // ---- activations as exact integers -------------------------------------------------------
-// Every group of 64 activations is scaled by its own power of two 2^f (its largest |x|
-// lands in [2^21, 2^22)) and rounded to the nearest integer: X = x * 2^f rounded,
-// |X| <= 2^22, the only rounding before the epilogue. X's two's-complement bytes are its
+// Every 64 activations are scaled by a power of two 2^f of their own (their largest |x|
+// lands in [2^22, 2^23)) and rounded to the nearest integer: X = x * 2^f rounded,
+// |X| < 2^23, the only rounding before the epilogue. X's two's-complement bytes are its
 // digits, X = b0 + 256 b1 + 65536 s2 with b0, b1 unsigned and s2 the signed third byte
 // (exact while |X| < 2^23). They go to LDS as the byte operands of v_dot4: per 8-element
 // block six dwords [byte p][even | odd], "even" holding elements 0, 2, 4, 6 and "odd" 1,
 // 3, 5, 7 -- the order in which a code dword's low and high nibbles present the weights.
 // Per half-group (32 elements) LDS also holds sum(X) (as a float) and 2^-f.
-constexpr int kBlockBytes = 24;  // one 8-element block: 3 digit planes x (even, odd) dwords
+// P = 4 digits instead of 3 (weight groups of 32, whose rows the FMA kernel summed before): the
+// largest |x| lands in [2^24, 2^25), so that only elements below a half of it are rounded at all and
+// sum(X) still fits an int. Measured rel L2 against 64-bit sums, normal activations, 896..9728
+// elements: P = 3 1.4e-7 to 1.8e-7, P = 4 0.9e-7 to 1.0e-7 (the FMA kernel 1.2e-7 to 1.3e-7).
+constexpr int block_bytes(int P) { return 8 * P; }  // one 8-element block: P digit planes x (even, odd) dwords
+constexpr int kBlockBytes = block_bytes(3);
 
-// Round to nearest (ties upward: floor(v + 0.5)), one instruction.
+// f for 64 activations with the largest |x| m; f <= 149 as in group_exponent (every finite x is a
+// whole multiple of 2^-149). m is raised by one bit of its mantissa, so that no X rounds up to 2^23,
+// and halved, so that it stays finite. The instruction gives 0 for the exponent of a zero, whose X
+// are 0 with any f, and of an infinity or a NaN, where group_unscale gives the result.
+template <int P>
+__device__ inline int set_exponent(float m) {
+    return min((P == 3 ? 22 : 24) - __builtin_amdgcn_frexp_expf(m * 0.50000006f), 149);
+}
+
+// Round to nearest, ties to even. (Ties are common at this width, and rounding them upward in one
+// instruction, v_cvt_rpi_i32_f32, adds up over a row: 2.1e-7 to 2.9e-7 at G = 64 and 2.8e-7 to 3.9e-7 at
+// G = 128 instead of P = 3's figures above. The launch takes the same time: 2560x9728 7.07 us, with
+// integer maxima in stage_x paying for the extra instruction.)
 __device__ inline int round_int(float v) {
     int r;
-    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(rintf(v)));  // saturates: an infinity is met by group_unscale
     return r;
 }
 
 // Thread t converts 16-byte chunk c = t + kSetThreads i (elements 4c .. 4c + 3) of every chunk
 // the rows read (c < C): the 16 chunks of a group are one DPP row (16 lanes), the 8
 // chunks of a half-group half of one.
+template <int P = 3>
 __device__ __forceinline__ void stage_x(float4 q, int c, int Kc, int C, unsigned char *xp, float2 *hs) {
     if (c >= Kc) q = make_float4(0.f, 0.f, 0.f, 0.f);  // past K: zeros
-    float m = fmaxf(fmaxf(abs_or_inf(q.x), abs_or_inf(q.y)), fmaxf(abs_or_inf(q.z), abs_or_inf(q.w)));
-    m = fmaxf(m, dpp_f<kDppXor1>(m));
-    m = fmaxf(m, dpp_f<kDppXor2>(m));
-    m = fmaxf(m, dpp_f<kDppHalfMirror>(m));
-    m = fmaxf(m, dpp_f<kDppMirror>(m));  // the group's largest |x| (inf if any is not finite), in all 16 lanes
-    const int f = group_exponent(m);
+    // magnitudes compared as integers: infinities and NaNs are above every finite value
+    const auto mag = [](float v) { return static_cast<int>(__float_as_uint(v) & 0x7FFFFFFFu); };
+    int mi = max(max(mag(q.x), mag(q.y)), max(mag(q.z), mag(q.w)));
+    mi = max(mi, dpp_i<kDppXor1>(mi));
+    mi = max(mi, dpp_i<kDppXor2>(mi));
+    mi = max(mi, dpp_i<kDppHalfMirror>(mi));
+    mi = max(mi, dpp_i<kDppMirror>(mi));
+    const float m = __int_as_float(mi);  // the largest |x| (not finite if any is not), in all 16 lanes
+    const int f = set_exponent<P>(m);
     // the value itself is scaled (2^f is not a finite float for f >= 128; x * 2^f is exact)
     const unsigned X0 = round_int(ldexpf(q.x, f)), X1 = round_int(ldexpf(q.y, f));
     const unsigned X2 = round_int(ldexpf(q.z, f)), X3 = round_int(ldexpf(q.w, f));
@@ -55,9 +76,9 @@ __device__ __forceinline__ void stage_x(float4 q, int c, int Kc, int C, unsigned
     sum += dpp_i<kDppHalfMirror>(sum);  // the half-group's sum(X), in its 8 lanes
     if (c >= C) return;
     // elements 4c + 0, 2 are "even" bytes 2 (c & 1) + 0, 1 of the block; 4c + 1, 3 "odd"
-    unsigned char *blk = xp + (c >> 1) * kBlockBytes + 2 * (c & 1);
+    unsigned char *blk = xp + (c >> 1) * block_bytes(P) + 2 * (c & 1);
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
+    for (int p = 0; p < P; ++p) {
         const unsigned sel = 0x0C0C0000u | ((4u + p) << 8) | p;  // byte p of the second, byte p of the first
         *reinterpret_cast<unsigned short *>(blk + 8 * p) = static_cast<unsigned short>(__builtin_amdgcn_perm(X2, X0, sel));
         *reinterpret_cast<unsigned short *>(blk + 8 * p + 4) =
@@ -67,23 +88,33 @@ __device__ __forceinline__ void stage_x(float4 q, int c, int Kc, int C, unsigned
 }
 
 // scale * 2^-f * (sum(q * X) - zero * sum(X)) over one half-group: the 16 code bytes cd,
-// the group header hd, the half-group's 24 operand dwords xv (4 blocks) and its
-// (sum(X), 2^-f). The digit sums are exact integers (v_dot4: unsigned for b0 and b1,
-// signed for s2); sum(q * X) = (a0 + 256 a1) + 65536 a2 is formed in fp32.
-__device__ __forceinline__ float half_group_int(const v4i &cd, unsigned hd, const unsigned (&xv)[24], float2 hs) {
+// the group header hd, the half-group's 8 P operand dwords xv (4 blocks) and its
+// (sum(X), 2^-f). The digit sums are exact integers (v_dot4: unsigned for the low digits,
+// signed for the top one); sum(q * X) = (a0 + 256 a1) + 65536 (a2 [+ 256 a3]) is formed in fp32.
+template <int P>
+__device__ __forceinline__ float half_group_int(const v4i &cd, unsigned hd, const unsigned (&xv)[8 * P], float2 hs) {
     unsigned a0 = 0, a1 = 0;
-    int a2 = 0;
+    int a2 = 0, a3 = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const unsigned d = static_cast<unsigned>(cd[j]);
         const unsigned lo = d & kNibbles, hi = (d >> 4) & kNibbles;
-        a0 = __builtin_amdgcn_udot4(lo, xv[6 * j + 0], a0, false);
-        a0 = __builtin_amdgcn_udot4(hi, xv[6 * j + 1], a0, false);
-        a1 = __builtin_amdgcn_udot4(lo, xv[6 * j + 2], a1, false);
-        a1 = __builtin_amdgcn_udot4(hi, xv[6 * j + 3], a1, false);
-        a2 = __builtin_amdgcn_sdot4(static_cast<int>(lo), static_cast<int>(xv[6 * j + 4]), a2, false);
-        a2 = __builtin_amdgcn_sdot4(static_cast<int>(hi), static_cast<int>(xv[6 * j + 5]), a2, false);
+        const unsigned *x = xv + 2 * P * j;
+        a0 = __builtin_amdgcn_udot4(lo, x[0], a0, false);
+        a0 = __builtin_amdgcn_udot4(hi, x[1], a0, false);
+        a1 = __builtin_amdgcn_udot4(lo, x[2], a1, false);
+        a1 = __builtin_amdgcn_udot4(hi, x[3], a1, false);
+        if constexpr (P == 3) {
+            a2 = __builtin_amdgcn_sdot4(static_cast<int>(lo), static_cast<int>(x[4]), a2, false);
+            a2 = __builtin_amdgcn_sdot4(static_cast<int>(hi), static_cast<int>(x[5]), a2, false);
+        } else {
+            a2 = static_cast<int>(__builtin_amdgcn_udot4(lo, x[4], static_cast<unsigned>(a2), false));
+            a2 = static_cast<int>(__builtin_amdgcn_udot4(hi, x[5], static_cast<unsigned>(a2), false));
+            a3 = __builtin_amdgcn_sdot4(static_cast<int>(lo), static_cast<int>(x[6]), a3, false);
+            a3 = __builtin_amdgcn_sdot4(static_cast<int>(hi), static_cast<int>(x[7]), a3, false);
+        }
     }
+    if constexpr (P == 4) a2 += 256 * a3;
     const float V = fmaf(static_cast<float>(a2), 65536.f, static_cast<float>(a0 + a1 * 256u));
     const float sc = half_bits(hd), z = half_bits(hd >> 16);
     // 2^-f times the exact integer sum first: for tiny activations (f > 126) 2^-f is subnormal and

@@ -72,7 +72,8 @@ struct I4Mat {
 };
 constexpr int kSetMaxMats = 8;  // matrices per set launch
 // n independent matvecs sharing a group size: one launch per kSetMaxMats matrices the set
-// kernel takes (G = 64, K % 4 == 0, K <= 10240, x 16-byte aligned), the others one by one.
+// kernel takes (G = 32, 64 or 128, K % 4 == 0, K <= 10240, x 16-byte aligned; G = 128: and not too many rows),
+// the others one by one.
 int launch_i4_matvec_set(int n, const I4Mat *mats, int group_size, hipStream_t stream);
 // The set kernel for a single or fused launch when every matrix takes it and its grid is small
 // enough to beat the MFMA kernels; kNotFused (nothing launched) otherwise.
@@ -92,7 +93,7 @@ struct SetPrologue {
 // The set kernel with a prologue for up to 3 matrices sharing x (mats[i].x equal, 16-byte aligned
 // like x2, d1, d2, nw and hout); kNotFused (nothing launched) when the set kernel does not take them.
 int launch_i4_matvec_set_pro(int n, const I4Mat *mats, int group_size, const SetPrologue &pro, hipStream_t stream);
-// Whether the set kernel takes rows of K elements at this group size (with x 16-byte aligned).
+// Whether the set kernel with a prologue takes rows of K elements at this group size (64; x 16-byte aligned).
 bool set_kernel_takes(int K, int group_size);
 // A decode layer's gate / up pair (same shape, same x) with the kind-2 prologue pro, as one launch
 // storing act = silu(gate) * up to gate.y (up.y is not written): each value has the bits of the
