@@ -75,3 +75,35 @@ def test_long_row_table_matches_oracle(gpu, orc, M, K):
         got, fin = dy.download(np.float32, M), np.isfinite(want)
         assert np.array_equal(np.isfinite(got), fin) and (entry0 is not None or fin.all())
         assert rel_l2(got[fin], want[fin]) <= 1e-5
+
+
+# Rows per wave change at 4, 8 and 32 rows per CU (256 CUs), separately for rows of one step (in_dim
+# <= 1024) and longer ones; the last two are the largest the rows kernel takes and one past it.
+@pytest.mark.parametrize("M,K", [(1024, 16), (1025, 16), (1027, 1024), (1026, 1040), (2051, 2064), (8193, 272),
+                                 (8194, 2048), (8191, 3088), (32768, 1024), (32769, 1024)])
+def test_rows_per_wave_give_the_bits_of_one_row_at_a_time(gpu, orc, M, K):
+    """Each row's bits do not depend on how many rows a wave takes: alone, as a set of two matrices and
+    (a sample of rows) in launches of few rows, aligned x or not."""
+    w, xs = gpu.synth_vq2(M, K, seed=M + K), gpu.synth_normal(K + 1, seed=K)
+    dw, dx = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(xs)
+    cb, idx = w[:2048], w[2048:].reshape(M, K // 4)
+    sample = np.unique(np.r_[0:8, M // 2:M // 2 + 8, M - 8:M])
+    few = gpu.DeviceBuffer.from_array(np.concatenate([cb, idx[sample].reshape(-1)]))
+    w2 = gpu.synth_vq2(40, 2048, seed=3)
+    x2 = gpu.synth_normal(2048, seed=4)
+    dw2, dx2, dy2 = gpu.DeviceBuffer.from_array(w2), gpu.DeviceBuffer.from_array(x2), gpu.DeviceBuffer(160)
+    for off in (0, 1):
+        x = xs[off:off + K]
+        ptr = dx.ptr + 4 * off
+        dy, dfew, dset = gpu.DeviceBuffer(4 * M), gpu.DeviceBuffer(4 * len(sample)), gpu.DeviceBuffer(4 * M)
+        gpu.matvec_vq2_dev(dw, ptr, dy, M, K)
+        gpu.matvec_vq2_dev(few, ptr, dfew, len(sample), K)
+        gpu.matvec_vq2_set_dev([(dw2, dx2, dy2, 40, 2048), (dw, ptr, dset, M, K)])
+        gpu.synchronize()
+        got = dy.download(np.float32, M)
+        want = orc.matvec_vq2(w, x, M, K, threads=16)
+        assert rel_l2(got, want) <= 1e-6, rel_l2(got, want)  # fp32 sums of K / 64 terms a lane and 64 lanes
+        assert np.array_equal(dset.download(np.float32, M), got)
+        assert rel_l2(dy2.download(np.float32, 40), orc.matvec_vq2(w2, x2, 40, 2048)) <= 1e-6
+        if M * K <= 4 * (8 << 20):
+            assert np.array_equal(dfew.download(np.float32, len(sample)), got[sample])

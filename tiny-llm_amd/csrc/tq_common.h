@@ -111,7 +111,7 @@ bool i4_matvec_amax_takes(const uint8_t *w, const float *x, float *y, int out_di
                           int cap);  // whether the call above would launch
 int launch_vq2_matvec(const uint8_t *w, const float *x, float *y, int out_dim, int in_dim, hipStream_t stream);
 // n independent VQ2 matvecs (I4Mat: weights, activations, output, shape) in as few launches as
-// the one-wave-per-row kernel allows; each output has the bits launch_vq2_matvec gives it.
+// the rows kernel allows; each output has the bits launch_vq2_matvec gives it.
 int launch_vq2_matvec_set(int n, const I4Mat *mats, hipStream_t stream);
 // The same with each matrix's activations BiIP-rotated first (scale may be null, sign not), in
 // one launch; kNotFused when that launch does not take the set.

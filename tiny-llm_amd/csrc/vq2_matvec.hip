@@ -4,7 +4,7 @@
 // reference's matvec_vq2_ref (kernels/matvec/matvec_vq2_ref.cpp:52-81), on the
 // layout [codebook 256 x 4 fp16 = 2048 B][out_dim x in_dim/4 uint8 indices].
 //
-// Five kernels:
+// Seven kernels (vq2_matvec_rows and row1 are one body):
 // - vq2_matvec_table (index rows 16-byte aligned, in_dim <= 1024, at least 256 rows per CU):
 //   per workgroup a table of every codebook entry's dot product with every 4-element block of
 //   x, built with fp32 MFMAs in LDS; a lookup is then one 4-byte LDS read and one add (see its
@@ -20,12 +20,11 @@
 //   byte load per index. A wave owns a tile of kRows rows and sweeps the row in
 //   steps of 64 lanes x 4 indices; each lane keeps the 16 activations of its 4
 //   indices in VGPRs and reuses them for all kRows rows.
-// - vq2_matvec_rows (index rows dword-aligned, at most kDirectLookups lookups): one wave per
-//   row and no LDS at all. A grid this small cannot amortise building a 64 KB codebook
-//   replica per workgroup, so every lookup is an 8-byte load of the fp16 entry from the
-//   2 KB codebook in global memory (it stays in each CU's L1 after the first touch). One
-//   launch serves up to kSetMaxMats matrices with their own activations
-//   (launch_vq2_matvec_set: a decoder layer's q/k/v or gate/up).
+// - vq2_matvec_rows, vq2_matvec_row1 (index rows dword-aligned, at most kRowsLookups lookups): 1, 2
+//   or 4 rows per wave, the fp16 codebook (2 KB) in LDS, 8 bytes a lookup. A grid this small cannot
+//   amortise building a 64 KB codebook replica per workgroup. One launch serves up to kSetMaxMats
+//   matrices with their own activations (launch_vq2_matvec_set: a decoder layer's q/k/v or gate/up).
+// - vq2_matvec_direct (the same, at most kDirectRowsPerCu rows per CU): one wave per row and no LDS.
 // All accumulate in fp32.
 
 #include "lane_sum.h"
@@ -255,13 +254,23 @@ __global__ __launch_bounds__(64 * kVq2Waves) void vq2_matvec_copies(const uint8_
     }
 }
 
-// ---- One wave per row, codebook entries gathered from global memory (small launches).
+// ---- A few rows per wave, codebook entries gathered from LDS (small launches).
 // Lane l takes index dwords l, l + 64, ... of the row (indices 4 b .. 4 b + 3) and their
-// activations; the 64 lane sums are added by a butterfly over the wave. Measured on MI355X
-// against vq2_matvec_copies: 896x896 2.5 vs 5.2 us, 3072x1024 3.3-3.6 vs 5.1-5.3 us (the
-// one-launch floor for its 0.8 MB is 3.3 us), 4864x896 4.1 vs 5.3, 2001x3056 4.7 vs 7.9; from
-// about 8M lookups (16384x2048, 32768x896) the replica kernel is faster.
-constexpr long long kDirectLookups = 4ll << 20;
+// activations; the 64 lane sums are added by a butterfly over the wave. A lookup is an 8-byte
+// LDS read of the fp16 entry: gathered from L1 instead (64 addresses an instruction, which the
+// texture unit takes one after the other) the lookups bounded every launch of more than a few
+// rows per CU. Measured on MI355X (cold weights, graph), L1 -> LDS, us: a 0.5B-sized layer's seven
+// matrices 11.1 -> 5.7, gate / up pair 6.2 -> 4.1, 4864x896 3.9 -> 3.3, 8192x1024 5.1 -> 3.6, 4096x2560
+// 6.3 -> 4.3, 1720x9728 10.3 -> 7.7; against the replica kernel at 9728x2560 8.5 -> 6.4, 16384x2048
+// 7.7 -> 6.1, 32768x896 6.8 -> 6.1, while 40000x896 (9M lookups) is 7.5 there and 7.8 here.
+// Up to kDirectRowsPerCu rows per CU one wave per row and no LDS is as fast or faster, us: 128x896
+// 2.00 against 2.05, 896x896 2.06 against 2.13, 1024x3072 3.57 against 3.66.
+// The bits of a row are the same in all three forms (direct, rows, staged).
+constexpr long long kDirectLookups = 4ll << 20;  // a set's and a staged launch's matrix
+constexpr long long kRowsLookups = 8ll << 20;    // a matrix alone
+constexpr int kDirectRowsPerCu = 4;
+constexpr int kRowWaves = 4;    // waves per workgroup (8: 896x896 2.25 us against 2.13, 2560x4096 5.9 against 5.1)
+constexpr int kRowStep = 1024;  // elements of a step of 64 lanes x 4 indices
 // A launch of this kernel serves up to kSetMaxMats matrices, each with its own activations
 // (a layer's q/k/v, gate/up, or rotated copies of x): workgroups are numbered matrix after
 // matrix and a workgroup finds its matrix with scalar compares against the kernel argument.
@@ -355,10 +364,11 @@ __device__ inline float vq2_row(const uint8_t *w, const float *x, int K, int row
     return sum_wave(acc);  // DPP and row swaps in registers, a fixed order
 }
 
-// One matrix per launch (32 bytes of kernel arguments: the set form's 8 records and their
-// selection took 4.0 against 3.5 us at 3072x1024).
+// One matrix of at most kDirectRowsPerCu rows per CU: nothing is staged, a wave's row starts at
+// once, and every lookup is an 8-byte load of the codebook in global memory (it stays in each
+// CU's L1 after the first touch).
 template <bool XALIGN>
-__global__ __launch_bounds__(256) void vq2_matvec_row1(const uint8_t *__restrict__ w, const float *__restrict__ x,
+__global__ __launch_bounds__(256) void vq2_matvec_direct(const uint8_t *__restrict__ w, const float *__restrict__ x,
                                                        float *__restrict__ y, int M, int K) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
@@ -366,13 +376,80 @@ __global__ __launch_bounds__(256) void vq2_matvec_row1(const uint8_t *__restrict
     if ((threadIdx.x & 63) == 0) y[row] = acc;
 }
 
-template <bool XALIGN>
-__global__ __launch_bounds__(256) void vq2_matvec_rows(Vq2SetArgs a) {
+// R rows per wave of one matrix, x from global memory, the codebook's fp16 entries in LDS. Row r of
+// a wave is (blk R + r) kRowWaves + wave. The codebook entry and the rows' first index dwords are
+// loaded before the barrier, a step's dwords while the step before is looked up, and the R rows
+// share each step's activations.
+template <bool XALIGN, int R>
+__device__ __forceinline__ void vq2_rows(const uint8_t *w, const float *x, float *y, int M, int K, int blk, uint2 *cbl) {
+    const int nb4 = K / (4 * kVq2Dim);  // index dwords per row
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned *idx = reinterpret_cast<const unsigned *>(w + kVq2CodebookBytes);
+    const uint2 cb = reinterpret_cast<const uint2 *>(w)[threadIdx.x & 255];
+    const unsigned *qrow[R];
+    unsigned q[R];
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = (blk * R + r) * kRowWaves + wave;
+        qrow[r] = idx + static_cast<size_t>(row < M ? row : 0) * nb4;
+        q[r] = qrow[r][min(lane, nb4 - 1)];
+        acc[r] = 0.f;
+    }
+    if (threadIdx.x < 256) cbl[threadIdx.x] = cb;
+    __syncthreads();
+    for (int d0 = 0; d0 < nb4; d0 += 64) {
+        const int d = d0 + lane;
+        const int dc = min(d, nb4 - 1), dn = min(d + 64, nb4 - 1);
+        float4 xv[4];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+            const float *xp = x + 16 * dc + 4 * jj;
+            xv[jj] = XALIGN ? *reinterpret_cast<const float4 *>(xp) : make_float4(xp[0], xp[1], xp[2], xp[3]);
+        }
+        unsigned qn[R] = {};
+        if (d0 + 64 < nb4) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) qn[r] = qrow[r][dn];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            uint2 c[4];
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj) c[jj] = cbl[(q[r] >> (8 * jj)) & 0xFFu];
+            const float v = vq2_accum(acc[r], c, xv);
+            acc[r] = d < nb4 ? v : acc[r];
+            q[r] = qn[r];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = (blk * R + r) * kRowWaves + wave;
+        const float v = sum_wave(acc[r]);  // DPP and row swaps in registers, a fixed order
+        if (lane == 0 && row < M) y[row] = v;
+    }
+}
+
+// One matrix per launch (32 bytes of kernel arguments: the set form's 8 records and their
+// selection took 4.0 against 3.5 us at 3072x1024).
+template <bool XALIGN, int R>
+__global__ __launch_bounds__(64 * kRowWaves) void vq2_matvec_row1(const uint8_t *__restrict__ w,
+                                                                  const float *__restrict__ x, float *__restrict__ y,
+                                                                  int M, int K) {
+    __shared__ uint2 cbl[256];
+    vq2_rows<XALIGN, R>(w, x, y, M, K, blockIdx.x, cbl);
+}
+
+// R, RL: rows per wave of the matrices with rows of one step (K <= kRowStep), and of the others.
+template <bool XALIGN, int R, int RL>
+__global__ __launch_bounds__(64 * kRowWaves) void vq2_matvec_rows(Vq2SetArgs a) {
+    __shared__ uint2 cbl[256];
     TQ_VQ2_SELECT(a, m, kSetMaxMats);
-    const int row = (static_cast<int>(blockIdx.x) - m.blk0) * 4 + (threadIdx.x >> 6);
-    if (row >= m.M) return;
-    const float acc = vq2_row<XALIGN>(m.w, m.x, m.K, row, threadIdx.x & 63);
-    if ((threadIdx.x & 63) == 0) m.y[row] = acc;
+    const int blk = static_cast<int>(blockIdx.x) - m.blk0;
+    if (m.K <= kRowStep)
+        vq2_rows<XALIGN, R>(m.w, m.x, m.y, m.M, m.K, blk, cbl);
+    else
+        vq2_rows<XALIGN, RL>(m.w, m.x, m.y, m.M, m.K, blk, cbl);
 }
 
 // The staged form: 8 waves, each taking RPW rows, so that a workgroup's activation build serves
@@ -532,28 +609,67 @@ __global__ __launch_bounds__(64 * kRotWaves) void vq2_matvec_staged(Vq2StagedArg
     }
 }
 
-// The matrix the one-wave-per-row kernel takes: index rows dword-aligned, at most
-// kDirectLookups lookups.
-bool rows_kernel_takes(const uint8_t *w, int out_dim, int in_dim) {
+// The matrix the rows kernels take: index rows dword-aligned, at most `lookups` lookups.
+bool rows_kernel_takes(const uint8_t *w, int out_dim, int in_dim, long long lookups = kDirectLookups) {
     return (in_dim % 16) == 0 && (reinterpret_cast<uintptr_t>(w) % 4) == 0 &&
-           static_cast<long long>(out_dim) * (in_dim / kVq2Dim) <= kDirectLookups;
+           static_cast<long long>(out_dim) * (in_dim / kVq2Dim) <= lookups;
 }
 
-int launch_rows(Vq2SetArgs &a, int n, int blocks, bool xalign, hipStream_t stream) {
-    if (n == 1) {
+template <bool XALIGN, int R, int RL>
+void launch_rows_r(Vq2SetArgs &a, int n, int blocks, hipStream_t stream) {
+    const Vq2Mat &m = a.m[0];
+    const dim3 grid(blocks), block(64 * kRowWaves);
+    if (n > 1)
+        hipLaunchKernelGGL((vq2_matvec_rows<XALIGN, R, RL>), grid, block, 0, stream, a);
+    else if (m.K > kRowStep)
+        hipLaunchKernelGGL((vq2_matvec_row1<XALIGN, RL>), grid, block, 0, stream, m.w, m.x, m.y, m.M, m.K);
+    else
+        hipLaunchKernelGGL((vq2_matvec_row1<XALIGN, R>), grid, block, 0, stream, m.w, m.x, m.y, m.M, m.K);
+}
+
+template <bool XALIGN, int R>
+void launch_rows_l(int RL, Vq2SetArgs &a, int n, int blocks, hipStream_t stream) {
+    RL == 4   ? launch_rows_r<XALIGN, R, 4>(a, n, blocks, stream)
+    : RL == 2 ? launch_rows_r<XALIGN, R, 2>(a, n, blocks, stream)
+              : launch_rows_r<XALIGN, R, 1>(a, n, blocks, stream);
+}
+
+template <bool XALIGN>
+void launch_rows_x(int R, int RL, Vq2SetArgs &a, int n, int blocks, hipStream_t stream) {
+    R == 4   ? launch_rows_l<XALIGN, 4>(RL, a, n, blocks, stream)
+    : R == 2 ? launch_rows_l<XALIGN, 2>(RL, a, n, blocks, stream)
+             : launch_rows_l<XALIGN, 1>(RL, a, n, blocks, stream);
+}
+
+// Rows per wave by the launch's rows per CU, short and long ones by themselves: more rows share
+// a workgroup's codebook and a step's activations, fewer fill the chip. Measured with 1 / 2 / 4, us: 1152x896
+// (qkv) 2.70 / 2.55 / 2.83, 4864x896 3.47 / 3.27 / 3.52, 8192x1024 4.33 / 3.66 / 3.64, gate / up
+// (9728 rows) 5.46 / 4.27 / 4.07; 2001x3056 3.88 / 4.08 / 4.79, 2560x4096 5.06 / 4.90 / 5.55,
+// 4096x2560 4.95 / 4.29 / 4.80, 9728x2560 9.58 / 6.84 / 6.37.
+int launch_rows(Vq2SetArgs &a, int n, bool xalign, hipStream_t stream) {
+    const int cus = device_cu_count();
+    long rows[2] = {0, 0};  // short, long
+    for (int k = 0; k < n; ++k) rows[a.m[k].K > kRowStep] += a.m[k].M;
+    if (n == 1 && a.m[0].M <= kDirectRowsPerCu * cus) {
         const Vq2Mat &m = a.m[0];
+        const dim3 grid((m.M + 3) / 4), block(256);
         if (xalign)
-            hipLaunchKernelGGL(vq2_matvec_row1<true>, dim3(blocks), dim3(256), 0, stream, m.w, m.x, m.y, m.M, m.K);
+            hipLaunchKernelGGL(vq2_matvec_direct<true>, grid, block, 0, stream, m.w, m.x, m.y, m.M, m.K);
         else
-            hipLaunchKernelGGL(vq2_matvec_row1<false>, dim3(blocks), dim3(256), 0, stream, m.w, m.x, m.y, m.M, m.K);
+            hipLaunchKernelGGL(vq2_matvec_direct<false>, grid, block, 0, stream, m.w, m.x, m.y, m.M, m.K);
         return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
+    }
+    const int RS = rows[0] >= 32L * cus ? 4 : rows[0] >= 4L * cus ? 2 : 1;
+    const int RL = rows[1] >= 32L * cus ? 4 : rows[1] >= 8L * cus ? 2 : 1;
+    int blocks = 0;
+    for (int k = 0; k < n; ++k) {
+        a.m[k].blk0 = blocks;
+        const int per = kRowWaves * (a.m[k].K > kRowStep ? RL : RS);
+        blocks += (a.m[k].M + per - 1) / per;
     }
     for (int k = n; k < kSetMaxMats; ++k) a.m[k] = a.m[n - 1];  // never selected (k >= n)
     a.n = n;
-    if (xalign)
-        hipLaunchKernelGGL(vq2_matvec_rows<true>, dim3(blocks), dim3(256), 0, stream, a);
-    else
-        hipLaunchKernelGGL(vq2_matvec_rows<false>, dim3(blocks), dim3(256), 0, stream, a);
+    xalign ? launch_rows_x<true>(RS, RL, a, n, blocks, stream) : launch_rows_x<false>(RS, RL, a, n, blocks, stream);
     return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
 }
 
@@ -935,10 +1051,10 @@ int launch_vq2_matvec(const uint8_t *w, const float *x, float *y, int out_dim, i
     if (!w || !x || !y) return kBadShape;  // nothing is launched on a null operand
     const int cus = device_cu_count();
     const bool aligned = (in_dim % 16) == 0 && (reinterpret_cast<uintptr_t>(w) % 4) == 0;
-    if (rows_kernel_takes(w, out_dim, in_dim)) {
+    if (rows_kernel_takes(w, out_dim, in_dim, kRowsLookups)) {
         Vq2SetArgs a{};
         a.m[0] = Vq2Mat{w, x, y, out_dim, in_dim, 0, nullptr, nullptr};
-        return launch_rows(a, 1, (out_dim + 3) / 4, (reinterpret_cast<uintptr_t>(x) & 15) == 0, stream);
+        return launch_rows(a, 1, (reinterpret_cast<uintptr_t>(x) & 15) == 0, stream);
     }
     if (in_dim % 64 == 0 && in_dim <= kTabMaxDim && (reinterpret_cast<uintptr_t>(w) % 16) == 0 &&
         static_cast<long long>(out_dim) >= static_cast<long long>(kTabMinRowsPerCu) * cus) {
@@ -987,7 +1103,7 @@ int launch_vq2_matvec(const uint8_t *w, const float *x, float *y, int out_dim, i
     return hipGetLastError() == hipSuccess ? kOk : kLaunchFailed;
 }
 
-// The matrices the one-wave-per-row kernel takes go into one launch per kSetMaxMats of them
+// The matrices the rows kernel takes go into one launch per kSetMaxMats of them
 // (a launch is closed early once it holds more than 2 kDirectLookups lookups, where the replica
 // kernel would be faster); any other matrix is launched alone by launch_vq2_matvec. Every row
 // gets the same bits as from launch_vq2_matvec.
@@ -997,7 +1113,7 @@ int launch_vq2_matvec_set(int n, const I4Mat *mats, hipStream_t stream) {
         if (mats[i].M < 1 || mats[i].K < kVq2Dim || mats[i].K % kVq2Dim || !mats[i].w || !mats[i].x || !mats[i].y)
             return kBadShape;
     Vq2SetArgs a{};
-    int nb = 0, blocks = 0;
+    int nb = 0;
     long long lookups = 0;
     bool xalign = true;
     for (int i = 0; i < n; ++i) {
@@ -1009,21 +1125,20 @@ int launch_vq2_matvec_set(int n, const I4Mat *mats, hipStream_t stream) {
         }
         const long long lk = static_cast<long long>(mt.M) * (mt.K / kVq2Dim);
         if (nb == kSetMaxMats || (nb > 0 && lookups + lk > 2 * kDirectLookups)) {
-            const int st = launch_rows(a, nb, blocks, xalign, stream);
+            const int st = launch_rows(a, nb, xalign, stream);
             if (st != kOk) return st;
-            nb = blocks = 0;
+            nb = 0;
             lookups = 0;
             xalign = true;
         }
-        a.m[nb++] = Vq2Mat{mt.w, mt.x, mt.y, mt.M, mt.K, blocks, nullptr, nullptr};
-        blocks += (mt.M + 3) / 4;
+        a.m[nb++] = Vq2Mat{mt.w, mt.x, mt.y, mt.M, mt.K, 0, nullptr, nullptr};
         lookups += lk;
         xalign = xalign && (reinterpret_cast<uintptr_t>(mt.x) & 15) == 0;
     }
-    return nb > 0 ? launch_rows(a, nb, blocks, xalign, stream) : kOk;
+    return nb > 0 ? launch_rows(a, nb, xalign, stream) : kOk;
 }
 
-// n VQ2 matvecs in ONE launch of the one-wave-per-row kernel with staged activations: the
+// n VQ2 matvecs in ONE launch of the rows kernel with staged activations: the
 // prologue pro (kind 1 or 2, shared by the matrices, which then share x and K; null for none),
 // then, where sign is given, each matrix's own BiIP rotation (rotate as launch_biip_rotate, the
 // block size shared by the launch). Each output has the bits of the separate swiglu /
