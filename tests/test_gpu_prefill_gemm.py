@@ -120,3 +120,14 @@ def test_k_slices_in_a_captured_graph(gpu, orc):
                 assert np.array_equal(g.view(np.uint32), y.download(np.float32, M * N).view(np.uint32)), rep
     finally:
         graph.close()
+
+
+# the few-token kernel's slices: one (short rows), chosen by estimated time, the fewest that their
+# length allows (49 steps: 7 of 7; 50: 8), and two rounds of workgroups (tall, short rows)
+@pytest.mark.parametrize("M,K,N", [(129, 60, 8), (896, 256, 8), (129, 448, 3), (300, 512, 32), (1, 3136, 8),
+                                   (127, 3140, 1), (896, 4864, 8), (129, 16384, 5), (70000, 132, 2)])
+def test_few_token_slices(gpu, orc, M, K, N):
+    w, x = gpu.synth_i4(M, K, 64, seed=M + K), gpu.synth_normal(K * N, seed=N)
+    got = matmul_dev(gpu, w, x, M, K, N, 64)
+    assert np.array_equal(got, matmul_dev(gpu, w, x, M, K, N, 64))  # one order of the slices
+    assert rel_l2(got, orc.matmul_i4(w, x, M, K, N, 64, threads=8)) <= 2e-3

@@ -932,19 +932,34 @@ bool skinny_applies(const float *x, int K, int N, int group_size) {
 struct SkinnyGeom {
     int tiles, T, KS, smax;
     size_t part_bytes;  // the partial products
+    size_t room;        // the partials of as many slices as may be taken: what a fixed workspace must hold
 };
 
-// About 1.9 workgroups per CU (all resident at once; measured on MI355X at 9728x2560x32: 6
-// slices of 6-7 steps beat 8 of 5, the reduction of fewer partials outweighing the longer
-// slices), at most kSkMaxSteps steps per slice and at most one slice per step.
+// At most about 1.9 workgroups per CU (all resident at once), kSkMaxSteps steps per slice and one
+// slice per step; among these the slices with the least estimated time: the tile's last
+// workgroup reads its KS partials of 16 KB alone, 0.33 us each, a step of a slice takes 0.28 us
+// (fitted on MI355X to 896x4864 with 70 / 37 / 22 / 11 slices: 30.0, 19.5, 14.6, 11.7 us). Filling the
+// chip instead, us -> this rule, 8 tokens: 896x896 10.1 -> 7.7, 4864x896 12.0 -> 8.3, 896x4864
+// 30.2 -> 11.7, 2560x4096 19.6 -> 12.0, 2048x2048 17.9 -> 9.4; 9728x2560 and 151936x896 the same.
 SkinnyGeom skinny_geom(int M, int K) {
     SkinnyGeom g;
     g.tiles = (M + kSkRows - 1) / kSkRows;
     g.T = (K + 63) / 64;
     const int cus = device_cu_count();
     const int ks = std::max((19 * cus + 5 * g.tiles) / (10 * g.tiles), (g.T + kSkMaxSteps - 1) / kSkMaxSteps);
-    g.KS = std::max(1, std::min(ks, g.T));
+    const int most = std::max(1, std::min(ks, g.T));
+    g.KS = most;
+    float best = 0.f;
+    for (int k = most; k >= 1 && (g.T + k - 1) / k <= kSkMaxSteps; --k) {
+        const long rounds = (static_cast<long>(g.tiles) * k + 2 * cus - 1) / (2 * cus);
+        const float cost = (k > 1 ? 0.33f * k : 0.f) + 0.28f * ((g.T + k - 1) / k) * rounds;
+        if (k == most || cost < best) {
+            best = cost;
+            g.KS = k;
+        }
+    }
     g.smax = (g.T + g.KS - 1) / g.KS;
+    g.room = static_cast<size_t>(g.tiles) * most * kSkTile * sizeof(float);
     g.part_bytes = static_cast<size_t>(g.tiles) * g.KS * kSkTile * sizeof(float);
     return g;
 }
@@ -1146,7 +1161,7 @@ int launch_i4_matmul_noalloc(const uint8_t *w, const float *x, float *y, int M, 
         // bits, so a call whose partials do not fit is refused rather than rerouted
         // (e.g. 151936x896 at up to 32 tokens: 1187 tiles x 2 slices x 16 KiB).
         const SkinnyGeom g = skinny_geom(M, K);
-        if (g.part_bytes > kNoAllocWorkBytes || static_cast<size_t>(g.tiles) * 8 > kNoAllocArrivalBytes)
+        if (g.room > kNoAllocWorkBytes || static_cast<size_t>(g.tiles) * 8 > kNoAllocArrivalBytes)
             return kNoScratch;
         if (!operands) return kBadShape;
         unsigned char *ws = nullptr;
