@@ -15,12 +15,15 @@
  *    in HBM, launched asynchronously on `stream` (a hipStream_t; NULL = the
  *    default stream). They return 0 or a negative TQHIP_E* code and never abort.
  *    Scratch: some launches need library-owned device scratch (the split-K
- *    matvec's exchange slots, the prefill GEMM's fp16 copy of X). Each
+ *    matvec's exchange slots, the prefill GEMM's fp16 copy of X and the partial
+ *    products of its K slices). Each
  *    (device, stream) has its own, grown on demand between launches (the
  *    stream is synchronised first), so calls on different streams never share
  *    it. Under the caller's own stream capture nothing is allocated: a call
  *    that would need more scratch than the stream already has returns
- *    TQHIP_EHIP (run it once eagerly on that stream first), and scratch that a
+ *    TQHIP_EHIP (run it once eagerly on that stream first; only the partial
+ *    products can be missing: the slices then run one after the other, with the
+ *    same bits), and scratch that a
  *    capture recorded is never freed, so the caller's graph stays valid.
  *
  * 3. Registry. The library carries its own copy of the reference registry for
@@ -141,9 +144,10 @@ int tqhip_matvec_vq2_set_dev(const tqhip_i4_mat *mats, int n, void *stream);
  * holds until the process ends; its last 64 KiB hold the few-token kernel's tile counters
  * (zero between calls). A call whose fp16 copy needs more than the rest
  * (((ceil(K/64)*64*2*N + 255) & ~255) + 4*N bytes, e.g. above 3261 tokens at K = 2560), or
- * whose few-token partial products do not fit (16 KiB per 128-row tile and K slice, e.g.
+ * whose few-token partial products may not fit (16 KiB per 128-row tile and K slice it may take, e.g.
  * 151936x896 at up to 32 tokens: 38.9 MB), returns TQHIP_ENOSCRATCH before launching
- * anything; no call is rerouted to another kernel. Group sizes that are not a
+ * anything; no call is rerouted to another kernel (K slices above 32 tokens run one after the
+ * other, with the same bits). Group sizes that are not a
  * multiple of 32 run one matvec per token, with kernels that need no scratch. All calls
  * on one GPU share the array: calls that overlap on one GPU (two streams, or two host
  * threads) race and must be ordered by the caller. */
