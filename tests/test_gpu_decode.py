@@ -275,3 +275,31 @@ def test_long_context_attention_matches_oracle(gpu, tmp_path, shape, positions):
         if i in first:
             assert np.array_equal(eng.logits().view(np.uint32), first[i].view(np.uint32)), i
     eng.close()
+
+
+# One tile and several parts; 16 and 8 value rows a load (head_dim 128 and 256), whose later loads of a
+# tile lie wholly past the last position, and waves whose tile does.
+@pytest.mark.parametrize("shape", [dict(n_heads=2, n_kv_heads=2, head_dim=64), dict(n_heads=3, n_kv_heads=1, head_dim=128),
+                                   dict(n_heads=2, n_kv_heads=1, head_dim=256)])
+def test_cache_rows_past_the_position_are_not_used(gpu, tmp_path, shape):
+    """A sequence whose every key and value is NaN (token 0: an infinite embedding scale) fills the
+    cache; after a reset each step of a finite sequence has the bits of an engine whose cache is new."""
+    print(f"[decode] non-finite cache tail {shape}", flush=True)
+    n, cfg = 330, dict(hidden=128, inter=256, vocab=50, layers=1, max_seq_len=330, tied=False, **shape)
+    img, _, tensors = tf.dense_i4_model(seed=3, **cfg)
+    at = bytes(img).index(tensors["model.embed_tokens.weight"][2][:36])  # token 0's first group
+    img[at:at + 2] = np.float16(np.inf).tobytes()
+    path = tmp_path / "m.tqwen"
+    path.write_bytes(bytes(img))
+    m = gpu.ModelFile(str(path))
+    used, new = gpu.DecodeEngine(m), gpu.DecodeEngine(m)
+    for _ in range(n):
+        used.step(0)
+    assert not np.isfinite(used.logits()).any()
+    used.reset()
+    for i, t in enumerate(np.random.default_rng(4).integers(1, 50, n)):
+        a, b = used.step(int(t)), new.step(int(t))
+        la, lb = used.logits(), new.logits()
+        assert np.isfinite(la).all() and a == b and np.array_equal(la.view(np.uint32), lb.view(np.uint32)), i
+    used.close()
+    new.close()

@@ -132,12 +132,11 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_split(
     const float *kh = kcache + static_cast<size_t>(kvh) * max_seq * HD;
     const float *vh = vcache + static_cast<size_t>(kvh) * max_seq * HD;
     // Rows below pos are read: row pos is written by this launch and the rows after it are not there
-    // yet. A lane past them reads the key row before pos, unused; the value rows go through a
-    // buffer that ends at row pos, past which a load gives 0.
+    // yet (or left by a longer sequence before a reset, and not finite then). A lane past them reads
+    // the key row before pos, unused; a tile's value rows go through a buffer that ends at row pos,
+    // past which a load gives 0. The scalar offset of a load stays within that buffer: the range
+    // check subtracts it from the buffer's size, and what a difference below zero does is not said.
     const int last_row = max(pos - 1, 0);
-    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(vh), static_cast<short>(0), static_cast<int>(4u * HD * static_cast<unsigned>(pos)),
-        0x00020000);
     constexpr int KS = HD > 128 ? 64 : HD;  // key elements held at once (the VGPRs' limit)
     float4 kreg[KS / 4];
     float vreg[VB][E];
@@ -146,16 +145,20 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_split(
 #pragma unroll
         for (int i = 0; i < KS / 4; ++i) kreg[i] = attn_ld4(kr + 4 * i);
     };
-    const auto load_values = [&](int r0) {
+    const auto load_values = [&](int t0, int b) {  // rows b VB .. of tile t0 / 64
+        const int bytes = 4 * HD * min(max(pos - t0, 0), kSplitTile);
+        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(vh) + static_cast<size_t>(t0) * HD, static_cast<short>(0), bytes, 0x00020000);
+        const int so = min(4 * HD * VB * b, bytes);
 #pragma unroll
         for (int u = 0; u < VB; ++u)
 #pragma unroll
             for (int e = 0; e < E; ++e)
-                vreg[u][e] = __uint_as_float(
-                    __builtin_amdgcn_raw_buffer_load_b32(vr, 4 * (u * HD + lane + 64 * e), 4 * HD * r0, 0));
+                vreg[u][e] =
+                    __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(vr, 4 * (u * HD + lane + 64 * e), so, 0));
     };
     load_keys(tile0 * kSplitTile, 0);  // (a wave past the sequence reads the last row, unused)
-    load_values(tile0 * kSplitTile);
+    load_values(tile0 * kSplitTile, 0);
     __builtin_amdgcn_sched_barrier(0);  // (the cache loads go out before the work below waits for q)
 
     // RoPE angles of element lane (+ 64 a) of the lower half; HD 64: lanes 32.. take that of lane - 32
@@ -201,7 +204,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_split(
         const int t0 = tile * kSplitTile;
         if (tile != tile0) {
             load_keys(t0, 0);
-            load_values(t0);
+            load_values(t0, 0);
         }
         float p4[4] = {};  // (four chains: one alone waits for each FMA)
         const auto dot_keys = [&](int k0) {
@@ -234,7 +237,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_split(
         m = m_new;
 #pragma unroll 1
         for (int b = 0; b < kSplitTile / VB; ++b) {
-            if (b > 0) load_values(t0 + b * VB);
+            if (b > 0) load_values(t0, b);
             float a2[2][E] = {};  // even and odd rows
 #pragma unroll
             for (int u = 0; u < VB; ++u) {
