@@ -7,6 +7,8 @@ fp32 where the reference sums in double, and its softmax is two-pass), and the
 engine's next token equal to the oracle's argmax wherever the oracle's top two
 logits are more than 1e-3 of the logit scale apart. Replays after reset are
 bit-identical."""
+import time
+
 import numpy as np
 import pytest
 
@@ -222,14 +224,16 @@ def test_errors(gpu, tmp_path):
         gpu.DecodeEngine(gpu.ModelFile(str(path)))
 
 
-# Where a step runs the split attention (from position 64 on): both sides of the switch, the first
-# and last position of a wave's tile of 64 and of a workgroup's 256, one and several heads per K/V
-# head, every head width, and a cache of more tiles than the grid has waves for.
+# Where a step runs the split attention (from position 64 or 160 on): both sides of the switch, the first
+# and last position of a wave's tile of 64, of a workgroup's 256 and of each grid of parts, one and
+# several heads per K/V head, every head width, more heads than eight parts of each are resident for
+# (grids of 4 and 8 parts), and a cache of more tiles than the grid has waves for.
 @pytest.mark.parametrize("shape,positions", [
     (dict(n_heads=2, n_kv_heads=2, head_dim=64), 400),
     (dict(n_heads=6, n_kv_heads=2, head_dim=64), 400),
     (dict(n_heads=7, n_kv_heads=1, head_dim=128, qk_norm=True, biases=False), 400),
     (dict(n_heads=2, n_kv_heads=1, head_dim=256, qk_norm=True), 330),
+    (dict(n_heads=40, n_kv_heads=2, head_dim=64), 1100),
     (dict(n_heads=2, n_kv_heads=1, head_dim=64), 33100),
 ])
 def test_long_context_attention_matches_oracle(gpu, tmp_path, shape, positions):
@@ -259,7 +263,8 @@ def test_long_context_attention_matches_oracle(gpu, tmp_path, shape, positions):
     eng = gpu.DecodeEngine(m)
     dec = Decoder(cfg, tensors, positions, exact_attention=False)
     dec.seen, dec.attention = {}, attend
-    check = {63, 64, 65, 127, 128, 129, 255, 256, 257, 319, 320, 321, 32767, 32768, 32769, 33023, 33024, positions - 1}
+    check = {63, 64, 65, 127, 128, 129, 159, 160, 161, 191, 192, 255, 256, 257, 319, 320, 321, 1023, 1024, 2047, 2048,
+             4095, 4096, 8191, 8192, 16383, 16384, 32767, 32768, 32769, 33023, 33024, positions - 1}
     tokens = [int(t) for t in np.random.default_rng(5).integers(0, 100, positions)]
     first = {}
     for i, t in enumerate(tokens):
@@ -303,3 +308,32 @@ def test_cache_rows_past_the_position_are_not_used(gpu, tmp_path, shape):
         assert np.isfinite(la).all() and a == b and np.array_equal(la.view(np.uint32), lb.view(np.uint32)), i
     used.close()
     new.close()
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(14, 2, 64), (32, 8, 128), (64, 8, 128), (3, 1, 256)])
+def test_steps_do_not_depend_on_the_cache_length(gpu, heads, kv_heads, head_dim):
+    """The same sequence in a cache of its own length and in one of 32768 positions: the same bits, in the
+    same time. (Half as long again is far outside what repeats differ by, and far below the 2.5 times
+    that a grid of workgroups for the whole cache took at 32 heads of 128.)"""
+    print(f"[decode] cache length {heads}x{head_dim}", flush=True)
+    n = 300
+    img, _, _ = tf.dense_i4_model(hidden=256, n_heads=heads, n_kv_heads=kv_heads, head_dim=head_dim, inter=256, vocab=50,
+                                  layers=4, seed=2, max_seq_len=32768)
+    m = gpu.ModelFile.from_image(img)
+    engines = [gpu.DecodeEngine(m, n), gpu.DecodeEngine(m, 32768)]
+    took = [[], []]
+    for rep in range(3):
+        for e in engines:
+            e.reset()
+        for i in range(n):
+            for e, t in zip(engines, took):
+                start = time.perf_counter()
+                e.step(i % 50)
+                t.append(time.perf_counter() - start)
+            if rep == 0:
+                a, b = (e.logits().view(np.uint32) for e in engines)
+                assert np.array_equal(a, b), i
+    short, long = (np.median(np.reshape(t, (3, n))[1:, 170:], axis=None) for t in took)
+    assert long <= 1.5 * short, (long, short)
+    for e in engines:
+        e.close()

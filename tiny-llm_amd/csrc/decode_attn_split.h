@@ -1,5 +1,5 @@
 // decode_attn_split.h -- a decode step's attention with the sequence split over workgroups, for
-// the engine's steps at long contexts (decode_engine.hip chooses by position).
+// the engine's steps at long contexts (from split_from(head_dim) positions on).
 //
 // attention_step (decode_attn.h) gives a query head one workgroup, so a step costs what one CU
 // takes to read the head's whole cache: 10 us at 250 positions, 24 at 1500, 46 at 3000 (14 heads
@@ -35,11 +35,39 @@ constexpr int kSplitTile = 64;        // positions per tile: one per lane
 constexpr int kSplitWaves = 4;        // waves of a workgroup: that many tiles side by side
 constexpr int kSplitMaxParts = 128;   // parts of a sequence (longer sequences: several tiles a wave)
 
-// Parts in the grid for a cache of max_seq positions: a multiple of 8, so that the heads that read
-// one part of a K/V head's cache land on one XCD and share its L2.
-inline int split_grid_parts(int max_seq) {
-    const int span = kSplitTile * kSplitWaves, parts = (max_seq + span - 1) / span;
-    return (std::min(parts, kSplitMaxParts) + 7) / 8 * 8;
+// Position from which a step runs the split attention. What it takes off a step's layer against
+// attention_step (us; the layer takes 20 to 35): 14 heads of 64 -1.7 at position 64, -0.3 at 152, 0.2 at 160, 1.3
+// at 240; 32 heads of 128 -3.7, -0.3, 0.4 and 3.2; 4 heads of 256, where one thread adds a dimension of every
+// value row, -1.5 at 48, 2.6 at 64, 44 at 240. What it loses is before the scores: attention_step's
+// first wave has its keys requested before the position is known.
+constexpr int split_from(int head_dim) { return head_dim == 256 ? 64 : 160; }
+
+constexpr int kSplitSpan = kSplitTile * kSplitWaves;  // positions of a workgroup whose waves take one tile each
+
+// Parts in the grid of steps up to `positions` positions: `first` times a power of two, enough for one
+// tile a wave, up to kSplitMaxParts. The engine keeps a graph per grid and a step takes the smallest
+// that covers its sequence: with one grid for the whole cache, 32 heads of 128 in a cache of 32768
+// positions took 78 us a layer at position 180 instead of 31 (a workgroup without positions still takes a
+// CU until it has read the position, and a CU holds one of these workgroups).
+inline int split_parts(int positions, int first) {
+    int parts = first;
+    while (parts < kSplitMaxParts && parts * kSplitSpan < positions) parts *= 2;
+    return parts;
+}
+// The smallest grid: 8 parts, so that the heads that read one part of a K/V head's cache land on one
+// XCD and share its L2 (14 heads of 64 at 180 positions: a step's layer takes 21.9 us, with one part and
+// the heads dealt over the XCDs 22.2), or with more heads the 4, 2 or 1 whose workgroups are resident
+// at once, one per CU (64 heads of 128 at 160 to 250 positions: 34 us with 4 parts, 46 with 8).
+inline int split_first_parts(int n_heads, int cus) {
+    int parts = 8;
+    while (parts > 1 && parts * n_heads > cus) parts /= 2;
+    return parts;
+}
+// Grid of `parts` parts: the first 2^shift (at most 8) of every head, then the next 8, so that parts
+// which the sequence does not reach go out last.
+inline int split_shift(int parts) { return parts >= 8 ? 3 : parts == 4 ? 2 : parts - 1; }
+inline dim3 split_grid(int n_heads, int parts) {
+    return dim3(n_heads << split_shift(parts), parts >> split_shift(parts));
 }
 // Floats of the partials of n_heads heads: per (head, part) HD outputs, then a record
 // {maximum, 0, sum as a double}.
@@ -93,7 +121,7 @@ __device__ inline void split_finish(float (&x)[HD / 64], const float *nw, const 
 
 template <int HD>
 __global__ __launch_bounds__(64 * kSplitWaves) void attention_split(
-    int heads_per_kv, int n_heads, int max_seq, float theta, float eps, float scale, const int *pos_ptr,
+    int heads_per_kv, int n_heads, int shift, int max_seq, float theta, float eps, float scale, const int *pos_ptr,
     const float *q, const float *k, const float *v, const float *qb, const float *kb, const float *vb, const float *qn,
     const float *kn, float *kcache, float *vcache, float *partial, unsigned *arrivals, float *out) {
     constexpr int E = HD / 64, A = (HD + 127) / 128, half = HD / 2, NW = kSplitWaves;
@@ -103,7 +131,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_split(
     __shared__ float ms[NW], ws[kSplitMaxParts];
     __shared__ double ls[NW];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int parts_grid = gridDim.x, part = blockIdx.x, head = blockIdx.y, kvh = head / heads_per_kv;
+    const int parts_grid = gridDim.y << shift, part = (blockIdx.y << shift) + (blockIdx.x & ((1 << shift) - 1));
+    const int head = blockIdx.x >> shift, kvh = head / heads_per_kv;
 
     // the raw q of the head and k and v of its group, their biases and norm weights (absent ones:
     // the projection itself, unused). None of these loads depends on the position, and all are

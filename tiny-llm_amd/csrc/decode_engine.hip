@@ -158,12 +158,6 @@ __global__ void step_begin_f32(const float *table, const int *host_io, int *io, 
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = table[base + i];
 }
 
-// Position from which a step runs the split attention (decode_attn_split.h). Measured per launch, 14
-// heads of 64, attention_step against it: 5.0 and 5.7 us up to position 63 (attention_step's first
-// wave has its keys requested before the position is known), 6.6 and 5.8 at 100, 8.2 and 6.3 at 190,
-// 10.2 and 6.8 at 250, 24 and 9.1 at 1500.
-constexpr int kSplitFrom = 64;
-
 // One workgroup per query head: attention_head (decode_attn.h) on the raw q / k / v
 // projections, biases added at entry.
 template <int HD>
@@ -331,11 +325,14 @@ struct Engine {
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    // The same step with its attention split over the sequence (decode_attn_split.h), for steps of
-    // more than kSplitFrom positions; absent (split_parts 0) where the cache is not longer than that.
-    hipGraph_t graph_long = nullptr;
-    hipGraphExec_t exec_long = nullptr;
-    int split_parts = 0;
+    // The same step with its attention split over the sequence (decode_attn_split.h), for positions from
+    // split_from(head_dim) on: one graph per grid of parts, each twice the one before, up to the cache's.
+    struct LongStep {
+        int parts;
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+    };
+    std::vector<LongStep> long_steps;
     float *split_partial = nullptr;
     unsigned *split_arrivals = nullptr;  // zero between launches
     bool eager = false;  // TQHIP_DECODE_EAGER=1: launch the step kernel by kernel (for profilers)
@@ -399,11 +396,16 @@ int mv_rotated_set(const Engine &e, int n, const uint8_t *const *w, float *const
     return e.pd == 4 ? launch_vq2_matvec_set(n, mats, s) : launch_i4_matvec_set(n, mats, e.gs, s);
 }
 
-// Whether the step at position pos runs the split attention.
-bool split_step(const Engine &e, int pos) { return e.split_parts > 0 && pos >= kSplitFrom; }
+// The split attention's step for position pos; null: attention_step's.
+const Engine::LongStep *long_step(const Engine &e, int pos) {
+    if (pos < split_from(e.c.head_dim)) return nullptr;
+    for (const Engine::LongStep &l : e.long_steps)
+        if (pos < l.parts * kSplitSpan) return &l;
+    return e.long_steps.empty() ? nullptr : &e.long_steps.back();
+}
 
-// split: the attention launches of the long-context step.
-int forward(Engine &e, bool split) {
+// parts: the grid of the split attention's launches, 0 for attention_step.
+int forward(Engine &e, int parts) {
     hipStream_t s = e.stream;
     const int H = e.c.hidden_size, I = e.c.intermediate_size;
     const float eps = e.c.rms_norm_eps;
@@ -461,19 +463,19 @@ int forward(Engine &e, bool split) {
             for (int j = 0; j < 3; ++j)
                 if ((st = mvr(e, w3[j], e.pd, e.normed, y3[j], d3[j], H, *r3[j], s)) != kOk) return st;
         }
-        if (split) {
+        if (parts) {
             auto attn = e.c.head_dim == 64 ? attention_split<64> : e.c.head_dim == 128 ? attention_split<128>
                                                                                        : attention_split<256>;
-            attn<<<dim3(e.split_parts, e.c.n_heads), 64 * kSplitWaves, 0, s>>>(
-                e.c.n_heads / e.c.n_kv_heads, e.c.n_heads, e.max_seq, e.c.rope_theta, e.c.rms_norm_eps, e.attn_scale,
-                e.dev_io, e.q, e.k, e.v, L.qb, L.kb, L.vb, L.qn, L.kn, kc, vc, e.split_partial, e.split_arrivals,
-                e.attn);
+            attn<<<split_grid(e.c.n_heads, parts), 64 * kSplitWaves, 0, s>>>(
+                e.c.n_heads / e.c.n_kv_heads, e.c.n_heads, split_shift(parts), e.max_seq, e.c.rope_theta,
+                e.c.rms_norm_eps, e.attn_scale, e.dev_io, e.q, e.k, e.v, L.qb, L.kb, L.vb, L.qn, L.kn, kc, vc,
+                e.split_partial, e.split_arrivals, e.attn);
         } else {
-        auto attn = e.c.head_dim == 64 ? attention_step<64> : e.c.head_dim == 128 ? attention_step<128>
-                                                                                  : attention_step<256>;
-        attn<<<e.c.n_heads, kAttnThreads, 0, s>>>(e.c.n_heads / e.c.n_kv_heads, e.max_seq, e.c.rope_theta,
-                                                  e.c.rms_norm_eps, e.attn_scale, e.dev_io, e.q, e.k, e.v, L.qb,
-                                                  L.kb, L.vb, L.qn, L.kn, kc, vc, e.attn);
+            auto attn = e.c.head_dim == 64 ? attention_step<64> : e.c.head_dim == 128 ? attention_step<128>
+                                                                                      : attention_step<256>;
+            attn<<<e.c.n_heads, kAttnThreads, 0, s>>>(e.c.n_heads / e.c.n_kv_heads, e.max_seq, e.c.rope_theta,
+                                                      e.c.rms_norm_eps, e.attn_scale, e.dev_io, e.q, e.k, e.v, L.qb,
+                                                      L.kb, L.vb, L.qn, L.kn, kc, vc, e.attn);
         }
         if ((st = mvr(e, L.o, e.pd, e.attn, e.o, H, e.q_dim, L.ro, s)) != kOk) return st;
         if (e.fused) {
@@ -535,9 +537,9 @@ int forward(Engine &e, bool split) {
 }
 
 // The step captured into a graph (the eager pass before it has sized the engine's scratch).
-int capture(Engine &e, bool split, hipGraph_t *graph, hipGraphExec_t *exec) {
+int capture(Engine &e, int parts, hipGraph_t *graph, hipGraphExec_t *exec) {
     if (hipStreamBeginCapture(e.stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return kLaunchFailed;
-    const int st = forward(e, split);
+    const int st = forward(e, parts);
     const hipError_t end = hipStreamEndCapture(e.stream, graph);
     if (st != kOk || end != hipSuccess) return st != kOk ? st : static_cast<int>(kLaunchFailed);
     return hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0) == hipSuccess ? kOk : kLaunchFailed;
@@ -545,7 +547,8 @@ int capture(Engine &e, bool split, hipGraph_t *graph, hipGraphExec_t *exec) {
 
 int eager_forward(Engine &e) {
     ScratchScope scope(e.scratch);
-    return forward(e, split_step(e, e.seq_len));
+    const Engine::LongStep *l = long_step(e, e.seq_len);
+    return forward(e, l ? l->parts : 0);
 }
 
 // The data-flow step: the layers and the final norm as one cooperative launch, then the lm_head
@@ -642,8 +645,10 @@ void release(Engine *e) {
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     if (e->exec) (void)hipGraphExecDestroy(e->exec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
-    if (e->exec_long) (void)hipGraphExecDestroy(e->exec_long);
-    if (e->graph_long) (void)hipGraphDestroy(e->graph_long);
+    for (const Engine::LongStep &l : e->long_steps) {
+        if (l.exec) (void)hipGraphExecDestroy(l.exec);
+        if (l.graph) (void)hipGraphDestroy(l.graph);
+    }
     scratch_set_free(e->scratch);
     if (e->arena) (void)hipFree(e->arena);
     if (e->host_io) (void)hipHostFree(e->host_io);
@@ -823,7 +828,9 @@ int create(void *model, int max_seq_len, std::string *err, Engine **out) {
     // [layer][k|v][kv_head][max_seq][head_dim], the argmax partials.
     e->layer_stride = static_cast<size_t>(c.n_kv_heads) * max_seq_len * c.head_dim;
     e->amax_blocks = (c.vocab_size + kArgmaxPerBlock - 1) / kArgmaxPerBlock;
-    e->split_parts = max_seq_len > kSplitFrom ? split_grid_parts(max_seq_len) : 0;
+    const int parts_first = split_first_parts(c.n_heads, device_cu_count());
+    const int parts_max = max_seq_len > split_from(c.head_dim) ? split_parts(max_seq_len, parts_first) : 0;
+    for (int parts = parts_first; parts <= parts_max; parts *= 2) e->long_steps.push_back({parts, nullptr, nullptr});
     const size_t counts[] = {H, H, static_cast<size_t>(e->q_dim), static_cast<size_t>(e->kv_dim),
                              static_cast<size_t>(e->kv_dim), static_cast<size_t>(e->q_dim), H, I, I, H, V,
                              2 * static_cast<size_t>(c.n_layers) * e->layer_stride,
@@ -835,8 +842,8 @@ int create(void *model, int max_seq_len, std::string *err, Engine **out) {
                              2 * static_cast<size_t>(e->kv_dim), 2 * static_cast<size_t>(e->q_dim), 2 * H, 2 * I,
                              2 * H,
                              // the split attention's partials and arrival counters
-                             e->split_parts ? split_partial_floats(c.n_heads, c.head_dim, e->split_parts) : 0,
-                             e->split_parts ? static_cast<size_t>(c.n_heads) : 0};
+                             parts_max ? split_partial_floats(c.n_heads, c.head_dim, parts_max) : 0,
+                             parts_max ? static_cast<size_t>(c.n_heads) : 0};
     float **slots[] = {&e->hidden, &e->normed, &e->q, &e->k, &e->v, &e->attn, &e->o, &e->gate, &e->up, &e->ffn,
                        &e->logits, &e->kv, &e->amax_v};
     constexpr int kSlots = 18 + kFlowVecs + 2;
@@ -901,12 +908,13 @@ int create(void *model, int max_seq_len, std::string *err, Engine **out) {
     // outside the capture; its KV rows are rewritten by the first real step.
     e->scratch = scratch_set_new();
     ScratchScope scope(e->scratch);
-    int rc = forward(*e, false);
+    int rc = forward(*e, 0);
     if (rc == kOk && hipStreamSynchronize(e->stream) != hipSuccess) rc = kLaunchFailed;
     const char *eager = std::getenv("TQHIP_DECODE_EAGER");
     e->eager = eager && eager[0] == '1';
-    if (rc == kOk && !e->eager) rc = capture(*e, false, &e->graph, &e->exec);
-    if (rc == kOk && !e->eager && e->split_parts) rc = capture(*e, true, &e->graph_long, &e->exec_long);
+    if (rc == kOk && !e->eager) rc = capture(*e, 0, &e->graph, &e->exec);
+    for (Engine::LongStep &l : e->long_steps)
+        if (rc == kOk && !e->eager) rc = capture(*e, l.parts, &l.graph, &l.exec);
     if (rc != kOk) {
         *err = "gpu engine: setting up the step graph failed";
         release(e);
@@ -951,7 +959,7 @@ int tqhip_decode_step(void *engine, int token_id) {
     if (!e || token_id < 0 || token_id >= e->c.vocab_size || e->seq_len >= e->max_seq) return kBadShape;
     e->host_io[0] = e->seq_len;
     e->host_io[1] = token_id;
-    const bool split = split_step(*e, e->seq_len);
+    const Engine::LongStep *split = long_step(*e, e->seq_len);
     if (e->flow && !split) {  // (the split attention's steps run through their graph)
         e->host_io[3] = static_cast<int>(++e->run);
         e->host_io[4] = 0;
@@ -975,7 +983,7 @@ int tqhip_decode_step(void *engine, int token_id) {
     // word (the logits were stored by the launch before it); past a bound, or if the word never
     // comes, the stream is synchronised, which reports a failed launch.
     __atomic_store_n(&e->host_io[2], -1, __ATOMIC_SEQ_CST);
-    if (e->eager ? eager_forward(*e) != kOk : hipGraphLaunch(split ? e->exec_long : e->exec, e->stream) != hipSuccess)
+    if (e->eager ? eager_forward(*e) != kOk : hipGraphLaunch(split ? split->exec : e->exec, e->stream) != hipSuccess)
         return kLaunchFailed;
     const auto t0 = std::chrono::steady_clock::now();
     int next = -1;
