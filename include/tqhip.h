@@ -139,7 +139,8 @@ int tqhip_matvec_vq2_set_dev(const tqhip_i4_mat *mats, int n, void *stream);
  * for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc). Same kernels and results as
  * tqhip_matmul_i4_dev, bit for bit. X's fp16 copy and the per-token scales (or, at up to
- * 32 tokens with group_size 64, the few-token kernel's partial products) go to a static
+ * 32 tokens with group_size 64 and rows of at most 114240 elements, the few-token kernel's
+ * partial products) go to a static
  * device array of TQHIP_NOALLOC_SCRATCH_BYTES (16 MiB) that every GPU the library runs on
  * holds until the process ends; its last 64 KiB hold the few-token kernel's tile counters
  * (zero between calls). A call whose fp16 copy needs more than the rest

@@ -131,3 +131,20 @@ def test_few_token_slices(gpu, orc, M, K, N):
     got = matmul_dev(gpu, w, x, M, K, N, 64)
     assert np.array_equal(got, matmul_dev(gpu, w, x, M, K, N, 64))  # one order of the slices
     assert rel_l2(got, orc.matmul_i4(w, x, M, K, N, 64, threads=8)) <= 2e-3
+
+
+# the longest row that the few-token kernel's slices cover (255 of 7 steps), and one past it, which
+# takes the tiled GEMM; the few-token call after it finds its counters zero
+@pytest.mark.parametrize("K", [114240, 114244, 131072])
+def test_rows_past_the_few_token_slices(gpu, orc, K):
+    M, N, G = 130, 3, 64
+    print(f"[few tokens] {M}x{K}x{N}", flush=True)
+    w, x = gpu.synth_i4(M, K, G, seed=K), gpu.synth_normal(K * N, seed=K + 1)
+    got = matmul_dev(gpu, w, x, M, K, N, G)
+    assert rel_l2(got, orc.matmul_i4(w, x, M, K, N, G, threads=16)) <= 2e-3
+    dw, dx, dy = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(4 * M * N)
+    assert gpu.matmul_i4_noalloc_dev(dw, dx, dy, M, K, N, G) == gpu.OK
+    gpu.synchronize()
+    assert np.array_equal(dy.download(np.float32, M * N), got)
+    w, x = gpu.synth_i4(896, 4864, G, seed=1), gpu.synth_normal(4864 * 8, seed=2)
+    assert rel_l2(matmul_dev(gpu, w, x, 896, 4864, 8, G), orc.matmul_i4(w, x, 896, 4864, 8, G, threads=16)) <= 2e-3

@@ -21,6 +21,7 @@
 // itself and splits K over workgroups (section 3 below).
 // Other group sizes: one i4 matvec per token column.
 
+#include "few_token_slices.h"
 #include "i4_lane.h"
 #include "tq_common.h"
 
@@ -313,7 +314,6 @@ __device__ __forceinline__ HalfOffsets half_offsets(int s, int G, int gb, int gr
 constexpr int kSplitNone = 0, kSplitParts = 1, kSplitSeq = 2;
 constexpr int kDeviceScope = 16;  // buffer cache policy: sc1 (device-scope coherent)
 constexpr int kL1Bypass = 1;      // buffer cache policy: sc0 (misses in the CU's L1, served by the XCD's L2)
-constexpr int kXccSlots = 14;     // slices whose writer's XCD the arrival counter carries
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 //   Partials are [tile][slice][wave][token block][float4][lane] (the MFMA's register order: every
@@ -349,12 +349,12 @@ __device__ inline bool add_parts(f16x (&acc)[WN], float *part, unsigned long lon
     wait_vm(0);       // this wave's partial stores have completed
     __syncthreads();  // and every other wave's
     if (threadIdx.x == 0) {
-        // bits 56..63: arrivals; bits 4 p .. 4 p + 3: 1 + the XCD of slice p's writer
+        // (the counter's layout: few_token_slices.h)
         const unsigned long long mine =
-            (1ull << 56) | (ks < kXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
+            (1ull << kArrivalShift) | (ks < kXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
         const unsigned long long prev =
             __hip_atomic_fetch_add(arrivals + tile, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool last = (prev >> 56) == static_cast<unsigned long long>(KS - 1);
+        const bool last = (prev >> kArrivalShift) == static_cast<unsigned long long>(KS - 1);
         if (last) __hip_atomic_store(arrivals + tile, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last_s = last;
         writers_s = prev;
@@ -668,10 +668,7 @@ __global__ __launch_bounds__(64 * NWV) void i4_matmul_direct(const uint8_t *__re
 //     other partials from that XCD's L2; the arrival counter (zero between launches: the
 //     last arrival resets it) carries each writer's XCD, so a partial written elsewhere is
 //     read at device scope instead.
-constexpr int kSkRows = 128;
-constexpr int kSkReduceBatch = 6; // partials the last arrival has in flight at once
-constexpr int kSkTile = kSkRows * 32;  // floats of one partial
-constexpr int kSkMaxSteps = 7;  // a row's slice (9 dwords a step) within one 64-lane DMA
+constexpr int kSkReduceBatch = 6;  // partials the last arrival has in flight at once
 
 template <int SMAX>
 __global__ __launch_bounds__(256) void i4_matmul_skinny(const uint8_t *__restrict__ w, const float *__restrict__ x,
@@ -819,12 +816,12 @@ __global__ __launch_bounds__(256) void i4_matmul_skinny(const uint8_t *__restric
         wait_vm(0);       // this wave's partial stores have completed
         __syncthreads();  // and every other wave's
         if (threadIdx.x == 0) {
-            // bits 56..63: arrivals; bits 4 p .. 4 p + 3: 1 + the XCD of slice p's writer
+            // (the counter's layout: few_token_slices.h)
             const unsigned long long mine =
-                (1ull << 56) | (ks < kXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
+                (1ull << kArrivalShift) | (ks < kXccSlots ? static_cast<unsigned long long>(xcc + 1) << (4 * ks) : 0ull);
             const unsigned long long prev =
                 __hip_atomic_fetch_add(arrivals + tile, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const bool last = (prev >> 56) == static_cast<unsigned long long>(KS - 1);
+            const bool last = (prev >> kArrivalShift) == static_cast<unsigned long long>(KS - 1);
             if (last) __hip_atomic_store(arrivals + tile, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             last_s = last;
             writers_s = prev;
@@ -924,45 +921,10 @@ int launch_direct(const uint8_t *w, const _Float16 *xh, const float *xinv, float
 }
 
 // The few-token kernel applies: G = 64, at most 32 tokens, whole 16-byte X loads (K % 4 == 0,
-// X 16-byte aligned) and the byte offsets of 128 rows within 31 bits.
+// X 16-byte aligned) and rows that its slices cover (whose 128 are then within 31-bit byte offsets).
 bool skinny_applies(const float *x, int K, int N, int group_size) {
     return group_size == 64 && N <= 32 && K % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-           static_cast<size_t>(kSkRows) * i4_row_bytes(K, 64) < (1ull << 31);
-}
-
-struct SkinnyGeom {
-    int tiles, T, KS, smax;
-    size_t part_bytes;  // the partial products
-    size_t room;        // the partials of as many slices as may be taken: what a fixed workspace must hold
-};
-
-// At most about 1.9 workgroups per CU (all resident at once), kSkMaxSteps steps per slice and one
-// slice per step; among these the slices with the least estimated time: the tile's last
-// workgroup reads its KS partials of 16 KB alone, 0.33 us each, a step of a slice takes 0.28 us
-// (fitted on MI355X to 896x4864 with 70 / 37 / 22 / 11 slices: 30.0, 19.5, 14.6, 11.7 us). Filling the
-// chip instead, us -> this rule, 8 tokens: 896x896 10.1 -> 7.7, 4864x896 12.0 -> 8.3, 896x4864
-// 30.2 -> 11.7, 2560x4096 19.6 -> 12.0, 2048x2048 17.9 -> 9.4; 9728x2560 and 151936x896 the same.
-SkinnyGeom skinny_geom(int M, int K) {
-    SkinnyGeom g;
-    g.tiles = (M + kSkRows - 1) / kSkRows;
-    g.T = (K + 63) / 64;
-    const int cus = device_cu_count();
-    const int ks = std::max((19 * cus + 5 * g.tiles) / (10 * g.tiles), (g.T + kSkMaxSteps - 1) / kSkMaxSteps);
-    const int most = std::max(1, std::min(ks, g.T));
-    g.KS = most;
-    float best = 0.f;
-    for (int k = most; k >= 1 && (g.T + k - 1) / k <= kSkMaxSteps; --k) {
-        const long rounds = (static_cast<long>(g.tiles) * k + 2 * cus - 1) / (2 * cus);
-        const float cost = (k > 1 ? 0.33f * k : 0.f) + 0.28f * ((g.T + k - 1) / k) * rounds;
-        if (k == most || cost < best) {
-            best = cost;
-            g.KS = k;
-        }
-    }
-    g.smax = (g.T + g.KS - 1) / g.KS;
-    g.room = static_cast<size_t>(g.tiles) * most * kSkTile * sizeof(float);
-    g.part_bytes = static_cast<size_t>(g.tiles) * g.KS * kSkTile * sizeof(float);
-    return g;
+           skinny_row_fits(K);
 }
 
 int launch_skinny(const uint8_t *w, const float *x, float *y, int M, int K, int N, const SkinnyGeom &g, float *part,
@@ -1013,14 +975,15 @@ TilePlan tile_plan(int M, int K, int N) {
                                {kTile128x32, 128, 32, 0.3f, 0.4f, 0.25f, 4.f, 0.25f},
                                {kTile128x64, 128, 64, 0.4f, 0.6f, 0.42f, 4.f, 0.45f},
                                {kTile256x96, 256, 96, 0.77f, 1.6f, 0.8f, 0.f, 0.f}};
-    constexpr int kMaxSlices = 32;
+    constexpr int kMostSlices = 32;
+    static_assert(kMostSlices <= kMaxSlices, "the arrival counter's count");
     TilePlan best{};
     float cost = 0.f;
     for (const Tile &t : kTiles) {
         // one token block: the 32-token tiles; more: the others (they share W loads among tokens)
         if ((N <= 32) != (t.bn == 32)) continue;
         const size_t tiles = static_cast<size_t>((M - 1) / t.bm + 1) * ((N - 1) / t.bn + 1);
-        for (int ks = 1; ks <= (t.split > 0.f ? std::min(kMaxSlices, steps) : 1); ++ks) {
+        for (int ks = 1; ks <= (t.split > 0.f ? std::min(kMostSlices, steps) : 1); ++ks) {
             const size_t n = (tiles * ks - 1) / cus + 1, bytes = ks > 1 ? tiles * ks * t.bm * t.bn * sizeof(float) : 0;
             const float step = n == 1 ? t.one : n == 2 ? t.two : t.many * static_cast<float>(n);
             const float c = static_cast<float>((steps - 1) / ks + 1) * step +
@@ -1161,7 +1124,7 @@ int launch_i4_matmul_noalloc(const uint8_t *w, const float *x, float *y, int M, 
         // launch_i4_matmul runs the few-token kernel here; another kernel would give other
         // bits, so a call whose partials do not fit is refused rather than rerouted
         // (e.g. 151936x896 at up to 32 tokens: 1187 tiles x 2 slices x 16 KiB).
-        const SkinnyGeom g = skinny_geom(M, K);
+        const SkinnyGeom g = skinny_geom(M, K, device_cu_count());
         if (g.room > kNoAllocWorkBytes || static_cast<size_t>(g.tiles) * 8 > kNoAllocArrivalBytes)
             return kNoScratch;
         if (!operands) return kBadShape;
@@ -1192,7 +1155,7 @@ int launch_i4_matmul(const uint8_t *w, const float *x, float *y, int M, int K, i
     if (M < 1 || K < 1 || N < 1 || group_size < 2 || (group_size & 1)) return kBadShape;
     if (!w || !x || !y) return kBadShape;  // nothing is launched on a null operand
     if (skinny_applies(x, K, N, group_size)) {
-        const SkinnyGeom g = skinny_geom(M, K);
+        const SkinnyGeom g = skinny_geom(M, K, device_cu_count());
         unsigned long long *slots = nullptr;  // zero between launches: the arrival counters
         int st = scratch_split_slots(stream, static_cast<size_t>(g.tiles), &slots);
         if (st != kOk) return st;
