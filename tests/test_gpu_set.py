@@ -279,3 +279,24 @@ def test_extreme_activations_by_group_size(gpu, orc, G):
         gpu.matvec_i4_dev(dw, gpu.DeviceBuffer.from_array(x), dy, M, K, G)
         gpu.synchronize()
         assert not np.isfinite(dy.download(np.float32, M)).any()
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_groups_of_32_at_any_weight_address(gpu, orc, offset):
+    """Weights that do not start on 4 bytes: the wave-per-row kernel (the same bits as its own entry
+    point), alone, as a pair and in a set."""
+    M, K, G = 70, 864, 32
+    w, x = gpu.synth_i4(M, K, G, seed=2), gpu.synth_normal(K, seed=3)
+    dw = gpu.DeviceBuffer.from_array(np.concatenate([np.zeros(offset, np.uint8), w, np.zeros(4, np.uint8)]))
+    dx, ys = gpu.DeviceBuffer.from_array(x), [gpu.DeviceBuffer(4 * M) for _ in range(5)]
+    p = dw.ptr + offset
+    gpu.lib().tqhip_matvec_i4_generic_dev(p, dx.ptr, ys[0].ptr, M, K, G, None)
+    gpu.matvec_i4_dev(p, dx, ys[1], M, K, G)
+    gpu.matvec_i4_set_dev(gpu.i4_set([(p, dx, ys[2], M, K)]), G)
+    gpu.lib().tqhip_matvec_pair_i4_dev(p, p, dx.ptr, ys[3].ptr, ys[4].ptr, M, K, G, None)
+    gpu.synchronize()
+    got = [y.download(np.float32, M) for y in ys]
+    want = orc.matvec_i4(w, x, M, K, G)
+    assert np.linalg.norm(got[0] - want) <= 1e-6 * np.linalg.norm(want)  # fp32 sums of 27 groups
+    for g in got[1:]:
+        assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))

@@ -258,10 +258,11 @@ __global__ __launch_bounds__(kSetThreads) void i4_matvec_glu(SetArgs<2> a) {
 }
 
 // Shape of a matrix in the set kernel, or -1 when the kernel does not take it:
-// G = 32, 64 or 128, K % 4 == 0 and x 16-byte aligned (whole 16-byte activation loads), K <= 10240.
+// G = 32, 64 or 128, K % 4 == 0 and x 16-byte aligned (whole 16-byte activation loads), K <= 10240; and
+// at G = 32, whose other kernel reads w by the byte from any address, w 4-byte aligned.
 int set_shape(const I4Mat &mt, int group_size) {
     if ((group_size != 64 && group_size != 32 && group_size != 128) || mt.K % 4 != 0 || mt.K > kSetMaxSlots * 64 * 32 ||
-        (reinterpret_cast<uintptr_t>(mt.x) & 15) != 0)
+        (reinterpret_cast<uintptr_t>(mt.x) & 15) != 0 || (group_size == 32 && (reinterpret_cast<uintptr_t>(mt.w) & 3) != 0))
         return -1;
     return mt.K <= 1024 ? 0 : (mt.K + 64 * 32 - 1) / (64 * 32);
 }
