@@ -300,3 +300,44 @@ def test_groups_of_32_at_any_weight_address(gpu, orc, offset):
     assert np.linalg.norm(got[0] - want) <= 1e-6 * np.linalg.norm(want)  # fp32 sums of 27 groups
     for g in got[1:]:
         assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("G", [32, 128])
+@pytest.mark.parametrize("M,K,peak,where", [(65, 864, 300, "tiny scales"), (65, 4864, 3000, "tiny scales"),
+                                            (130, 9728, 1e6, "tiny scales"), (65, 2080, 3000, "zero weights")])
+def test_an_outlier_costs_only_its_own_group(gpu, orc, G, M, K, peak, where):
+    """One activation of every second group far above the others, where it counts for little: its group's
+    scales are tiny, or its own weights are 0. Each row is held to its rounding. Groups of 32: x to 2^-31 of
+    the largest |x| of its group, and then one rounding of each half-group's value; groups of 128: x to
+    2^-23 of the largest of its 64, and the half-group's sums, formed in fp32 (3 roundings of their
+    terms); then the slots, the wave sum and the stores' at most 12 roundings of the values."""
+    rng = np.random.default_rng(K + G)
+    groups = -(-K // G)
+    w = gpu.synth_i4(M, K, G, seed=K).reshape(M, groups, 4 + G // 2)
+    x = rng.standard_normal(K).astype(np.float32)
+    x[::2 * G] = peak
+    head = w[:, :, :4].copy().view(np.float16)  # scale, zero
+    if where == "tiny scales":
+        head[:, ::2, 0] = 6e-8
+    else:
+        head[:, ::2, 1] = np.rint(head[:, ::2, 1].astype(np.float32))
+        w[:, ::2, 4] = (w[:, ::2, 4] & 0xF0) | head[:, ::2, 1].astype(np.uint8)
+    w[:, :, :4] = head.view(np.uint8)
+    w = np.ascontiguousarray(w).reshape(-1)
+    dw, dx, dy = gpu.DeviceBuffer.from_array(w), gpu.DeviceBuffer.from_array(x), gpu.DeviceBuffer(4 * M)
+    gpu.matvec_i4_dev(dw, dx, dy, M, K, G)
+    gpu.synchronize()
+    pad = -K % 64
+    wd = np.pad(orc.dequant_i4_matrix_f64(w, M, K, G), ((0, 0), (0, pad)))
+    xp = np.pad(x.astype(np.float64), (0, pad))
+    scale = np.pad(np.repeat(np.abs(head[:, :, 0].astype(np.float64)), G, axis=1)[:, :K], ((0, 0), (0, pad)))
+    block, step = (32, 2.0**-31) if G == 32 else (64, 2.0**-23)
+    largest = np.repeat(np.abs(xp).reshape(-1, block).max(1), block)
+    halves = np.abs((wd * xp).reshape(M, -1, 32).sum(2)).sum(1)
+    bound = step * (np.abs(wd) @ largest) + 12 * 2.0**-24 * halves
+    if G == 128:
+        bound += 3 * 2.0**-24 * 30 * (scale @ np.abs(xp))
+    err = np.abs(dy.download(np.float32, M) - wd @ xp)
+    assert np.all(err <= bound), f"worst row err/bound = {float(np.max(err / bound)):.3f}"
+    print(f"[outlier] G {G} {M}x{K} {where}: rel L2 {np.linalg.norm(err) / np.linalg.norm(wd @ xp):.2e}, "
+          f"worst err/bound {float(np.max(err / bound)):.2f}", flush=True)

@@ -149,7 +149,7 @@ __device__ __attribute__((always_inline)) bool flow_rows(const RowsJob &j, const
     const int C = 8 * U;
     const int Kc = j.K / 4;
     unsigned char *xp = lds;
-    float2 *hs = reinterpret_cast<float2 *>(lds + (C / 2) * kBlockBytes);
+    XSum<3> *hs = reinterpret_cast<XSum<3> *>(lds + (C / 2) * kBlockBytes);
 
     // 1. the rows' weights, all of them, before anything waits
     const int half = S == 0 ? lane >> 5 : 0, u = S == 0 ? lane & 31 : lane;
@@ -246,7 +246,7 @@ __device__ __attribute__((always_inline)) bool flow_rows(const RowsJob &j, const
         for (int i = 0; i < NX; ++i) xq[i] = rms_apply(xq[i], scale, pw[i]);
     }
 #pragma unroll
-    for (int i = 0; i < NX; ++i) stage_x(xq[i], t + kSetThreads * i, Kc, C, xp, hs);
+    for (int i = 0; i < NX; ++i) stage_x<3>(xq[i], t + kSetThreads * i, Kc, C, xp, hs);
     __syncthreads();
 
     // 4. the row sums (set_rows' order), then the tagged outputs
@@ -267,7 +267,7 @@ __device__ __attribute__((always_inline)) bool flow_rows(const RowsJob &j, const
             xv[4 * k + 2] = v[2];
             xv[4 * k + 3] = v[3];
         }
-        const float2 h = hs[ru];
+        const XSum<3> h = hs[ru];
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const float v = half_group_int<3>(cd[r * NS + sl], hd[r * NS + sl], xv, h);
@@ -552,7 +552,7 @@ bool flow_shapes_ok(int H, int q_dim) {
 // norm's sums. The layer records follow at that offset (flow_lds_table + layers * 128 bytes).
 size_t flow_lds_table(int H, int q_dim, int I) {
     const int kmax = H > q_dim ? (H > I ? H : I) : (q_dim > I ? q_dim : I);
-    const size_t rows = static_cast<size_t>(2 * ((kmax + 63) / 64)) * (4 * kBlockBytes + 8);
+    const size_t rows = static_cast<size_t>(2 * ((kmax + 63) / 64)) * (4 * kBlockBytes + sizeof(XSum<3>));
     const size_t attn = 2 * sizeof(AttnShared);
     return (std::max(rows, attn) + 255) / 256 * 256;
 }

@@ -22,9 +22,9 @@
 //     activation digits, exact before a per-half-group fp32 epilogue.
 // The same kernel serves single-matrix and pair / qkv launches of decode size
 // (launch_i4_matvec_set_fit), so a matrix gives the same bits alone or in a set.
-// Numerics: the only rounding before the epilogue is x -> X (at most 2^-23 of the largest |x| of
-// 64, groups of 32: 2^-25); measured rel L2 1.4e-7 to 1.8e-7 (groups of 32: 1.0e-7) against the
-// double-accumulating reference (kernels/matvec/matvec_i4_ref.cpp:45-103).
+// Numerics: the only rounding before the epilogue is x -> X (at most 2^-23 of the largest |x| of 64;
+// groups of 32: 2^-31 of the largest of 32); measured rel L2 1.6e-7 to 1.8e-7 (groups of 32: 0.6e-7 to 0.8e-7)
+// against the double-accumulating reference (kernels/matvec/matvec_i4_ref.cpp:45-103).
 // Groups of 32 and 128 took a wave-per-row FMA kernel and the split-K and register-path MFMA
 // kernels before; measured cold, us: 128: 896x4864 8.0 -> 5.0, 2560x4096 8.1 -> 4.4, 9728x2560
 // 8.4 -> 7.4, 2560x9728 12.5 -> 7.1; 32: 4864x896 13.5 -> 4.2, 9728x2560 63 -> 9.4, 151936x2560
@@ -62,8 +62,8 @@ constexpr int set_digits(int G) { return G == 32 ? 4 : 3; }
 // workgroup 0 storing the sum to hout), with its operands in pro. GLU: every row of m is computed
 // together with the same row of w2 (a matrix of m's shape reading the same x), and the row's
 // output is swiglu(m row, w2 row), as the separate outputs would give it in a SwiGLU prologue.
-// G: the weights' group size. The activations' exponents are per 64 elements whatever G is, and a
-// lane's half-group of 32 elements lies in one weight group, so G only moves the addresses.
+// G: the weights' group size. The activations' exponents are per 64 elements (G = 32: 32), and a
+// lane's half-group of 32 elements lies in one weight group, so otherwise G only moves the addresses.
 template <int S, int R, int XM, bool GLU = false, int G = 64>
 __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char *lds, const SetPrologue &pro,
                                          const uint8_t *w2 = nullptr) {
@@ -82,7 +82,7 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
     constexpr int P = set_digits(G);
     const int C = 8 * U;                                 // 16-byte activation chunks the rows read
     unsigned char *xp = lds;                                              // C / 2 blocks of operands
-    float2 *hs = reinterpret_cast<float2 *>(lds + (C / 2) * block_bytes(P));  // U (sum(X), 2^-f)
+    XSum<P> *hs = reinterpret_cast<XSum<P> *>(lds + (C / 2) * block_bytes(P));  // U of them
 
     // 1. the activations first: chunk t + kSetThreads i, clamped to the last one (zeroed past K
     // in stage_x). (Plain 16-byte loads: with a 16-byte buffer load whose elements are used
@@ -196,7 +196,7 @@ __device__ __forceinline__ void set_rows(const SetMat &m, int blk, unsigned char
             xv[4 * k + 2] = v[2];
             xv[4 * k + 3] = v[3];
         }
-        const float2 h = hs[ru];
+        const XSum<P> h = hs[ru];
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const float v = half_group_int<P>(cd[r * NS + sl], hd[r * NS + sl], xv, h);
@@ -332,7 +332,9 @@ int launch_set(const I4Mat *mats, const int *shape, int n, int group_size, hipSt
     }
     for (int k = n; k < kSetMaxMats; ++k) a.m[k] = a.m[n - 1];  // never selected (k >= n)
     a.n = n;
-    const size_t lds = static_cast<size_t>(umax) * (4 * block_bytes(set_digits(group_size)) + 8);  // the widest row's operands
+    // the widest row's operands
+    const size_t lds = static_cast<size_t>(umax) * (group_size == 32 ? 4 * block_bytes(4) + sizeof(XSum<4>)
+                                                                     : 4 * block_bytes(3) + sizeof(XSum<3>));
     const dim3 grid(blocks), block(kSetThreads);
     const int xm = pro ? pro->kind : 0;
     if (group_size != 64) {  // (prologue launches are G = 64 only)
@@ -445,7 +447,7 @@ int launch_i4_matvec_glu(const I4Mat &gate, const I4Mat &up, int group_size, con
     a.pro = pro;
     const int per = shape == 0 ? 2 * kSetWaves : kSetWaves;  // rows (pairs) per workgroup
     const dim3 grid((gate.M + per - 1) / per), block(kSetThreads);
-    const size_t lds = static_cast<size_t>(2 * ((gate.K + 63) / 64)) * (4 * kBlockBytes + 8);
+    const size_t lds = static_cast<size_t>(2 * ((gate.K + 63) / 64)) * (4 * kBlockBytes + sizeof(XSum<3>));
     switch (shape) {
         case 0: hipLaunchKernelGGL((i4_matvec_glu<0, 2>), grid, block, lds, stream, a); break;
         case 1: hipLaunchKernelGGL((i4_matvec_glu<1, 2>), grid, block, lds, stream, a); break;
