@@ -107,3 +107,16 @@ def test_rows_per_wave_give_the_bits_of_one_row_at_a_time(gpu, orc, M, K):
         assert rel_l2(dy2.download(np.float32, 40), orc.matvec_vq2(w2, x2, 40, 2048)) <= 1e-6
         if M * K <= 4 * (8 << 20):
             assert np.array_equal(dfew.download(np.float32, len(sample)), got[sample])
+
+
+# few tokens of long rows, which one matvec per token gives faster: up to 2, 4, 6 and 8 tokens at these
+# lengths, and one token more
+@pytest.mark.parametrize("M,K,most", [(33, 1024, 2), (130, 2560, 4), (70, 9728, 6), (5, 32768, 8)])
+def test_few_tokens_of_long_rows(gpu, orc, M, K, most):
+    w, x = gpu.synth_vq2(M, K, seed=M), gpu.synth_normal(K * (most + 1), seed=K)
+    each = np.concatenate([gpu.matvec_vq2(w, x[n * K:(n + 1) * K], M, K) for n in range(most + 1)])
+    for n in (2, most):
+        assert np.array_equal(gpu.matmul_vq2(w, x[:n * K], M, K, n).view(np.uint32), each[:n * M].view(np.uint32)), n
+    got = gpu.matmul_vq2(w, x, M, K, most + 1)
+    assert not np.array_equal(got, each)  # the matrix launch: other sums
+    assert rel_l2(got, product(orc, w, x, M, K, most + 1)) <= 1e-5

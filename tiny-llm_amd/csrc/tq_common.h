@@ -124,7 +124,8 @@ int launch_vq2_matvec_set_rot(int n, const I4Mat *mats, const float *const *scal
 int launch_vq2_matvec_set_pro(int n, const I4Mat *mats, const float *const *scale, const float *const *sign,
                               int block_size, const SetPrologue *pro, hipStream_t stream);
 // Y[M,N] = W X over N tokens (x[n*K + k], y[n*M + m]) in fp32, one launch; kNotFused (nothing
-// launched) for an activation array that is not 16-byte aligned or a size past its offsets.
+// launched) for an activation array that is not 16-byte aligned, a size past its offsets, or few tokens
+// of long rows, which one matvec per token gives faster.
 int launch_vq2_matmul(const uint8_t *w, const float *x, float *y, int M, int K, int N, hipStream_t stream);
 bool vq2_set_takes(int n, const int *M, int K, int xm);
 int launch_i4_embed_rows(const uint8_t *embed, const int *rows, int n, int dim, int group_size, float *out,

@@ -153,13 +153,21 @@ __global__ __launch_bounds__(kMmThreads) void vq2_matmul(const uint8_t *__restri
     }
 }
 
+// Whether one matvec per token is faster than the matrix launch: a wave takes every eighth chunk of its row
+// one after the other, 6.4 ns an element of the row whatever the number of tokens up to 32, and a matvec
+// takes 2.2 us and 0.7 ns an element. A call on host arrays of 896 rows, us, matrix launch and matvecs:
+// 2 tokens of 896 elements 25 and 23, of 2560 46 and 36, of 9728 87 and 47; 6 tokens of 2560 55 and 59, of 4864 69
+// and 68, of 9728 99 and 90; 8 tokens of 9728 105 and 113. (Rows that are not a multiple of 16 elements: 4 us
+// and more a matvec, 26 and 33 at 2 tokens of 1004.)
+bool matvecs_are_faster(int K, int N) { return K % 16 == 0 && N * (2200.0 + 0.7 * K) < 6.4 * K; }
+
 }  // namespace
 
 int launch_vq2_matmul(const uint8_t *w, const float *x, float *y, int M, int K, int N, hipStream_t stream) {
     if (M < 1 || N < 1 || K < kVq2Dim || K % kVq2Dim || !w || !x || !y) return kBadShape;
     // 16-byte activation loads, 32-bit offsets within 32 index rows, and at most 65535 token tiles
     if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(w) & 3) || K >= (1 << 26) ||
-        N > 32 * 65535)
+        N > 32 * 65535 || matvecs_are_faster(K, N))
         return kNotFused;
     const bool aligned = K % 16 == 0;
     const int vec_y = M % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
