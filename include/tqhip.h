@@ -328,9 +328,10 @@ void tqhip_model_free(void *model);                   /* frees the HBM copy too 
  * and, with TQHIP_DECODE_FLOW=1 in the environment at create, run a step as one cooperative
  * launch of the whole layer stack whose phases wait for each other's outputs through tagged
  * vectors in HBM, then the lm_head and the argmax ("flow"; the default is the graph, which is
- * as fast or faster on MI355X). The flow step gives the graph step's logits bit for bit; if
- * one of its waits runs out (100 ms), the engine reports it on stderr, runs that token through
- * the graph and keeps to the graph. */
+ * as fast or faster on MI355X). That holds for the first 160 positions (head_dim 256: 64); the steps
+ * after them run through the graph, with their attention split over the sequence. The flow step gives
+ * the graph step's logits bit for bit; if one of its waits runs out (100 ms), the engine reports it on
+ * stderr, runs that token through the graph and keeps to the graph. */
 int tqhip_decode_create(void *model, int max_seq_len, char *err, int err_len, void **engine);
 int tqhip_decode_step(void *engine, int token_id);
 void tqhip_decode_reset(void *engine);      /* back to position 0 (KvCache::reset) */
@@ -338,7 +339,7 @@ void tqhip_decode_destroy(void *engine);
 const float *tqhip_decode_logits(const void *engine);
 int tqhip_decode_seq_len(const void *engine);
 /* How the engine runs a step (no counterpart in the reference): TQHIP_DECODE_FUSED |
- * TQHIP_DECODE_FLOW | TQHIP_DECODE_EAGER bits, -1 for a null engine. */
+ * TQHIP_DECODE_FLOW (at the positions that it covers) | TQHIP_DECODE_EAGER bits, -1 for a null engine. */
 #define TQHIP_DECODE_FUSED 1
 #define TQHIP_DECODE_FLOW 2
 #define TQHIP_DECODE_EAGER 4
