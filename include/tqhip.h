@@ -328,7 +328,7 @@ void tqhip_model_free(void *model);                   /* frees the HBM copy too 
  * and, with TQHIP_DECODE_FLOW=1 in the environment at create, run a step as one cooperative
  * launch of the whole layer stack whose phases wait for each other's outputs through tagged
  * vectors in HBM, then the lm_head and the argmax ("flow"; the default is the graph, which is
- * as fast or faster on MI355X). That holds for the first 160 positions (head_dim 256: 64); the steps
+ * as fast or faster on MI355X). That holds for the first 160 positions (224 with wider heads); the steps
  * after them run through the graph, with their attention split over the sequence. The flow step gives
  * the graph step's logits bit for bit; if one of its waits runs out (100 ms), the engine reports it on
  * stderr, runs that token through the graph and keeps to the graph. */

@@ -131,11 +131,11 @@ def test_flow_wait_out_of_time_falls_back_to_the_graph(gpu, tmp_path, monkeypatc
 
 # positions from which a step's attention is split over the sequence: the data-flow kernel has no such
 # form, and those steps run through the graph
-@pytest.mark.parametrize("case,first", [("qwen25_0p5b_3layers", 160), ("qwen3_qknorm_hd128", 160), ("head_dim256", 64)])
+@pytest.mark.parametrize("case,first", [("qwen25_0p5b_3layers", 160), ("qwen3_qknorm_hd128", 224), ("head_dim256", 224)])
 def test_flow_hands_long_contexts_to_the_graph(gpu, tmp_path, monkeypatch, case, first):
     print(f"[flow] past position {first} {case}", flush=True)
     m, cfg, _ = open_model(gpu, tmp_path, case)
-    flow, graph = engines(gpu, m, monkeypatch, max_seq=200)
+    flow, graph = engines(gpu, m, monkeypatch, max_seq=240)
     tokens = [(13 * i + 5) % cfg["vocab_size"] for i in range(first + 8)]
     for _ in range(2):  # a reset takes the engine back to the data-flow step
         same_steps(flow, graph, tokens, cfg["vocab_size"], case)

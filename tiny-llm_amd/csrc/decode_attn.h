@@ -11,12 +11,14 @@
 // softmax, sum of p * v). Every head of a group computes the new k / v itself and uses its
 // own copy at position pos, so no head reads a cache row another workgroup is writing.
 //
-// Latency is the cost here (14 heads at Qwen2.5-0.5B), so the memory round trips are
-// overlapped: thread t's key row for position t (head_dim <= 128) and the first eight value
-// rows of its slice are issued at entry, and the RoPE angles are computed while they are in
-// flight. Thread j scores position j of a chunk of up to 4096 positions; the softmax over a
-// chunk is max / exp / sum, and across chunks the running max rescales the partial sums.
-// Thread t accumulates dimension t % hd over every (256 / hd)-th position, in position order.
+// The sequence has at most kAttnPositions positions (longer ones: decode_attn_split.h). Latency is the
+// cost here (14 heads at Qwen2.5-0.5B), so the memory round trips are overlapped: thread t's key row
+// for position t (head_dim <= 128) and the first eight value rows of its slice are issued at entry, and
+// the RoPE angles are computed while they are in flight. Thread t scores position t; then max / exp /
+// sum. Thread t accumulates dimension t % hd over every (256 / hd)-th position, in position order.
+// (One pass over so many positions, and the step's own key put into its thread's row before the scores:
+// a step's layer at position 40 takes 18.6 us with 14 heads of 64, 23.3 with 32 of 128 and 24.9 with 4 of 256;
+// with chunks of 4096 positions and a case of its own for that key 18.9, 25.2 and 34.3.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -29,7 +31,7 @@ namespace tqhip {
 namespace {
 
 constexpr int kAttnThreads = 256;
-constexpr int kAttnChunk = 4096;  // scores of one chunk of positions in LDS
+constexpr int kAttnPositions = 224;  // at most a position per thread
 constexpr int kAttnMaxHd = 256;
 
 // One head's LDS.
@@ -37,7 +39,7 @@ struct AttnShared {
     __attribute__((aligned(16))) float qs[kAttnMaxHd];
     __attribute__((aligned(16))) float ks[kAttnMaxHd];
     float vs[kAttnMaxHd];
-    float sc[kAttnChunk];
+    float sc[kAttnPositions];
     float part[kAttnThreads];
     float norm_scale[2];
     double dred[kAttnThreads / 64];
@@ -116,7 +118,7 @@ __device__ inline bool attention_head(AttnShared &S, int t, int head, int heads_
     // it (but below max_seq) are read and never used. The other waves' key rows go out after q / k /
     // v, once the position is known, so that a long cache is not read beyond the sequence.
     float4 kreg[kPrefetchKey ? HD / 4 : 1];
-    const bool key_pre = kPrefetchKey && t < seq && t != pos && t < kAttnChunk;
+    const bool key_pre = kPrefetchKey && t < seq && t != pos;
     if constexpr (kPrefetchKey) {
         if (t < 64) {  // (wave-uniform) the other waves' rows go out once q / k / v are in, below
             const float *kr = kh + static_cast<size_t>(t < max_seq ? t : 0) * hd;
@@ -223,102 +225,79 @@ __device__ inline bool attention_head(AttnShared &S, int t, int head, int heads_
         attn_st(vcache + (static_cast<size_t>(kvh) * max_seq + pos) * hd + t, S.vs[t]);
     }
 
-    float m = -INFINITY, l = 0.0f, acc = 0.0f;
     const float4 *q4 = reinterpret_cast<const float4 *>(S.qs);
-    for (int c0 = 0; c0 < seq; c0 += kAttnChunk) {
-        const int len = min(kAttnChunk, seq - c0);
-        for (int j = t; j < len; j += kAttnThreads) {
-            const int p = c0 + j;
-            float dot = 0.0f;
-            if (kPrefetchKey && p == t && key_pre) {
+    const float4 *k4 = reinterpret_cast<const float4 *>(S.ks);  // this step's own key
+    float score = -INFINITY;
+    if constexpr (kPrefetchKey) {
+        if (t == pos) {
 #pragma unroll
-                for (int i = 0; i < HD / 4; ++i) {
-                    const float4 a = q4[i], b = kreg[kPrefetchKey ? i : 0];
-                    dot += a.x * b.x;
-                    dot += a.y * b.y;
-                    dot += a.z * b.z;
-                    dot += a.w * b.w;
-                }
-            } else if (p == pos) {  // this step's own key, in LDS
-                const float4 *kr = reinterpret_cast<const float4 *>(S.ks);
-#pragma unroll
-                for (int i = 0; i < HD / 4; ++i) {
-                    const float4 a = q4[i], b = kr[i];
-                    dot += a.x * b.x;
-                    dot += a.y * b.y;
-                    dot += a.z * b.z;
-                    dot += a.w * b.w;
-                }
-            } else {
-                const float *kr = kh + static_cast<size_t>(p) * hd;
-#pragma unroll
-                for (int i = 0; i < HD / 4; ++i) {
-                    const float4 a = q4[i], b = attn_ld4(kr + 4 * i);
-                    dot += a.x * b.x;
-                    dot += a.y * b.y;
-                    dot += a.z * b.z;
-                    dot += a.w * b.w;
-                }
-            }
-            S.sc[j] = dot * scale;
+            for (int i = 0; i < HD / 4; ++i) kreg[i] = k4[i];
         }
-        // Each thread reduces only the scores it wrote; the value sums read the others' after
-        // attn_sum's barrier. fred and dred are each written once per chunk, and the chunk ends
-        // with a barrier.
-        float cmax = -INFINITY;
-        for (int j = t; j < len; j += kAttnThreads) cmax = fmaxf(cmax, S.sc[j]);
-        cmax = attn_max(cmax, S.fred, t);
-        const float m_new = fmaxf(m, cmax);
-        double csum = 0.0;
-        for (int j = t; j < len; j += kAttnThreads) {
-            const float p = expf(S.sc[j] - m_new);
-            S.sc[j] = p;
-            csum += p;
+    }
+    if (t < seq) {
+        float dot = 0.0f;
+        const auto add = [&](const float4 a, const float4 b) {
+            dot += a.x * b.x;
+            dot += a.y * b.y;
+            dot += a.z * b.z;
+            dot += a.w * b.w;
+        };
+        if constexpr (kPrefetchKey) {
+#pragma unroll
+            for (int i = 0; i < HD / 4; ++i) add(q4[i], kreg[i]);
+        } else if (t == pos) {
+#pragma unroll
+            for (int i = 0; i < HD / 4; ++i) add(q4[i], k4[i]);
+        } else {
+            const float *kr = kh + static_cast<size_t>(t) * hd;
+#pragma unroll
+            for (int i = 0; i < HD / 4; ++i) add(q4[i], attn_ld4(kr + 4 * i));
         }
-        csum = attn_sum(csum, S.dred, t);
-        const float rescale = expf(m - m_new);
-        l = l * rescale + static_cast<float>(csum);
-        acc = acc * rescale;
-        // The slice's positions j = slice, slice + slices, ... < len, added to acc in position
-        // order (acc + p * v each). Branch-free, eight positions at a time: their LDS reads and
-        // cache loads all go out before the first add (with a branch per position each LDS read
-        // was waited for before the next was issued), reads past the chunk are clamped to its
-        // last score, and the terms of positions past it are dropped by a select.
-        const float vpos = S.vs[d];  // position pos: this step's own value row, from LDS
-        int j = slice;
-        if (c0 == 0) {  // the first NV positions of the slice, loaded ahead
-            float scv[NV];
+        score = dot * scale;
+    }
+    const float m = attn_max(score, S.fred, t);
+    double sum = 0.0;
+    if (t < seq) {
+        const float p = expf(score - m);
+        S.sc[t] = p;
+        sum = p;
+    }
+    const float l = static_cast<float>(attn_sum(sum, S.dred, t));  // (its barrier: the others' probabilities are there)
+    // The slice's positions j = slice, slice + slices, ... < seq, added to acc in position
+    // order (acc + p * v each). Branch-free, eight positions at a time: their LDS reads and
+    // cache loads all go out before the first add (with a branch per position each LDS read
+    // was waited for before the next was issued), reads past the sequence are clamped to its
+    // last score, and the terms of positions past it are dropped by a select.
+    const float vpos = S.vs[d];  // position pos: this step's own value row, from LDS
+    float acc = 0.0f;
+    {  // the first NV positions of the slice, loaded ahead
+        float scv[NV];
 #pragma unroll
-            for (int u = 0; u < NV; ++u) scv[u] = S.sc[min(slice + u * slices, len - 1)];
+        for (int u = 0; u < NV; ++u) scv[u] = S.sc[min(slice + u * slices, pos)];
 #pragma unroll
-            for (int u = 0; u < NV; ++u) {
-                const int jj = slice + u * slices;
-                const float term = scv[u] * (jj == pos ? vpos : vreg[u]);
-                acc = jj < len ? acc + term : acc;
-            }
-            j = slice + NV * slices;
+        for (int u = 0; u < NV; ++u) {
+            const int j = slice + u * slices;
+            const float term = scv[u] * (j == pos ? vpos : vreg[u]);
+            acc = j < seq ? acc + term : acc;
         }
-        for (; j < len; j += 8 * slices) {
-            float vb8[8], sc8[8];
+    }
+    for (int j0 = slice + NV * slices; j0 < seq; j0 += 8 * slices) {
+        float vb8[8], sc8[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int jj = j + u * slices, p = c0 + jj;
-                // rows past the chunk and row pos (being written by this step) are not read: row 0
-                // instead, whose term is dropped (pos > 0 whenever a position past the first
-                // NV exists)
-                const bool use = jj < len && p != pos;
-                vb8[u] = attn_ld(vh + static_cast<size_t>(use ? p : 0) * hd + d);
-                sc8[u] = S.sc[min(jj, len - 1)];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int jj = j + u * slices;
-                const float term = sc8[u] * (c0 + jj == pos ? vpos : vb8[u]);
-                acc = jj < len ? acc + term : acc;
-            }
+        for (int u = 0; u < 8; ++u) {
+            const int j = j0 + u * slices;
+            // rows past the sequence and row pos (being written by this step) are not read: row 0
+            // instead, whose term is dropped (pos > 0 whenever a position past the first
+            // NV exists)
+            vb8[u] = attn_ld(vh + static_cast<size_t>(j < pos ? j : 0) * hd + d);
+            sc8[u] = S.sc[min(j, pos)];
         }
-        m = m_new;
-        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int j = j0 + u * slices;
+            const float term = sc8[u] * (j == pos ? vpos : vb8[u]);
+            acc = j < seq ? acc + term : acc;
+        }
     }
     S.part[t] = acc;
     __syncthreads();

@@ -35,12 +35,13 @@ constexpr int kSplitTile = 64;        // positions per tile: one per lane
 constexpr int kSplitWaves = 4;        // waves of a workgroup: that many tiles side by side
 constexpr int kSplitMaxParts = 128;   // parts of a sequence (longer sequences: several tiles a wave)
 
-// Position from which a step runs the split attention. What it takes off a step's layer against
-// attention_step (us; the layer takes 20 to 35): 14 heads of 64 -1.7 at position 64, -0.3 at 152, 0.2 at 160, 1.3
-// at 240; 32 heads of 128 -3.7, -0.3, 0.4 and 3.2; 4 heads of 256, where one thread adds a dimension of every
-// value row, -1.5 at 48, 2.6 at 64, 44 at 240. What it loses is before the scores: attention_step's
-// first wave has its keys requested before the position is known.
-constexpr int split_from(int head_dim) { return head_dim == 256 ? 64 : 160; }
+// Position from which a step runs the split attention, and what a step's layer takes there and nearby, us,
+// attention_step against it: 14 heads of 64 19.2 and 21.0 at 64, 21.0 and 21.6 at 152, 21.7 and 21.6 at 160, 23.4 and 22.2
+// at 240; 32 heads of 128 24.0 and 29.6 at 64, 31.2 and 31.4 at 216, 32.0 and 31.5 at 224; 4 heads of 256 26.4 and
+// 37.7 at 64, 41.4 and 41.6 at 224, 42.1 and 41.8 at 232. What it loses is before the scores:
+// attention_step's first wave has its keys requested before the position is known.
+constexpr int split_from(int head_dim) { return head_dim == 64 ? 160 : kAttnPositions; }
+static_assert(split_from(64) <= kAttnPositions && split_from(128) <= kAttnPositions, "attention_step's positions");
 
 constexpr int kSplitSpan = kSplitTile * kSplitWaves;  // positions of a workgroup whose waves take one tile each
 
