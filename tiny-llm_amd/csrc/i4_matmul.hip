@@ -17,7 +17,7 @@
 //      accumulation).
 //      fp16 and bf16 MFMA run at the same rate on gfx950; fp16 keeps 8x
 //      finer rounding of both operands.
-// Up to 32 tokens at G = 64 (16-byte aligned X, K % 4 == 0): one launch that converts X
+// Up to 32 tokens at G = 64 (16-byte aligned X, K % 4 == 0, K <= 114240): one launch that converts X
 // itself and splits K over workgroups (section 3 below).
 // Other group sizes: one i4 matvec per token column.
 
@@ -881,18 +881,6 @@ __global__ __launch_bounds__(256) void i4_matmul_skinny(const uint8_t *__restric
     }
 }
 
-// Raises fn's dynamic-LDS limit to what the CU's 160 KB leaves beside its static LDS
-// (once per kernel; `limit` caches the figure).
-int raise_lds_limit(const void *fn, size_t &limit) {
-    hipFuncAttributes attr{};
-    if (hipFuncGetAttributes(&attr, fn) != hipSuccess || attr.sharedSizeBytes >= 160 * 1024) return kLaunchFailed;
-    const size_t cap = 160 * 1024 - attr.sharedSizeBytes;
-    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(cap)) != hipSuccess)
-        return kLaunchFailed;
-    limit = cap;
-    return kOk;
-}
-
 // K slices of a call and where their partials go (part null: kSplitSeq).
 struct Slices {
     int KS;
@@ -905,12 +893,8 @@ int launch_direct(const uint8_t *w, const _Float16 *xh, const float *xinv, float
                   int rb, const Slices &sl, hipStream_t stream) {
     constexpr int BN = 32 * WN, BM = 32 * NWV;
     const auto kernel = i4_matmul_direct<GT, WN, S, NWV, SPLIT>;
-    const size_t lds = static_cast<size_t>(S) * BN * 128;
-    static size_t limit = 0;
-    if (lds > 64 * 1024 && limit == 0) {
-        if (raise_lds_limit(reinterpret_cast<const void *>(kernel), limit) != kOk) return kLaunchFailed;
-    }
-    if (lds > 64 * 1024 && lds > limit) return kTooLarge;
+    constexpr size_t lds = static_cast<size_t>(S) * BN * 128;
+    static_assert(lds <= 64 * 1024, "the dynamic LDS that a launch may take without raising its limit");
     if (static_cast<size_t>(BM) * rb + static_cast<size_t>(Kp) * 2 * BN >= (1ull << 31)) return kTooLarge;
     dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN);
     if (SPLIT == kSplitParts) grid = dim3((grid.x * grid.y + 7) / 8 * 8 * sl.KS);
