@@ -228,12 +228,14 @@ def test_errors(gpu, tmp_path):
 # Where a step runs the split attention (from position 160 or 224 on): both sides of the switch, the first
 # and last position of a wave's tile of 64, of a workgroup's 256 and of each grid of parts, one and
 # several heads per K/V head, every head width, more heads than eight parts of each are resident for
-# (grids of 4 and 8 parts), and a cache of more tiles than the grid has waves for.
+# (grids of 4 and 8 parts), more parts than the last arrival combines in one round (16 at head_dim 128, 8
+# at 256), and a cache of more tiles than the grid has waves for (several tiles a wave).
 @pytest.mark.parametrize("shape,positions", [
     (dict(n_heads=2, n_kv_heads=2, head_dim=64), 400),
     (dict(n_heads=6, n_kv_heads=2, head_dim=64), 400),
-    (dict(n_heads=7, n_kv_heads=1, head_dim=128, qk_norm=True, biases=False), 400),
-    (dict(n_heads=2, n_kv_heads=1, head_dim=256, qk_norm=True), 330),
+    (dict(n_heads=7, n_kv_heads=1, head_dim=128, qk_norm=True, biases=False), 4400),
+    (dict(n_heads=2, n_kv_heads=1, head_dim=256, qk_norm=True), 2400),
+    (dict(n_heads=1, n_kv_heads=1, head_dim=256), 33100),
     (dict(n_heads=40, n_kv_heads=2, head_dim=64), 1100),
     (dict(n_heads=2, n_kv_heads=1, head_dim=64), 33100),
 ])
@@ -265,7 +267,7 @@ def test_long_context_attention_matches_oracle(gpu, tmp_path, shape, positions):
     dec = Decoder(cfg, tensors, positions, exact_attention=False)
     dec.seen, dec.attention = {}, attend
     check = {63, 64, 65, 127, 128, 129, 159, 160, 161, 191, 192, 223, 224, 225, 255, 256, 257, 319, 320, 321, 1023, 1024, 2047, 2048,
-             4095, 4096, 8191, 8192, 16383, 16384, 32767, 32768, 32769, 33023, 33024, positions - 1}
+             2303, 2304, 4095, 4096, 4351, 4352, 8191, 8192, 16383, 16384, 32767, 32768, 32769, 33023, 33024, positions - 1}
     tokens = [int(t) for t in np.random.default_rng(5).integers(0, 100, positions)]
     first = {}
     for i, t in enumerate(tokens):
