@@ -119,9 +119,9 @@ typedef struct tqhip_i4_mat {
  * vectors). No counterpart in the reference, whose runtime issues a layer as separate
  * registry calls (runtime/qwen_forward_token.cpp:401, 458, 639, 658 through
  * kernels/dispatch.h:151-175): this is the "matvec set per layer" as one launch. Every
- * matrix with group_size 64, in_dim % 4 == 0, in_dim <= 10240 and x 16-byte aligned goes
- * into one launch per 8 such matrices; any other runs through tqhip_matvec_i4_dev's
- * kernels. Each output has the same bits as the lane kernels of tqhip_matvec_i4_dev give
+ * matrix with group_size 32, 64 or 128, in_dim % 4 == 0, in_dim <= 10240 and x 16-byte
+ * aligned (group_size 32: w 4-byte aligned too; 128: not too many rows) goes into one launch
+ * per 8 such matrices; any other runs through tqhip_matvec_i4_dev's kernels. Each output has the same bits as the lane kernels of tqhip_matvec_i4_dev give
  * it where those run (rows up to 1024 wide on small grids, up to 6144 wide on very small
  * ones). mats is read during the call. */
 int tqhip_matvec_i4_set_dev(const tqhip_i4_mat *mats, int n, int group_size, void *stream);
@@ -147,8 +147,8 @@ int tqhip_matvec_vq2_set_dev(const tqhip_i4_mat *mats, int n, void *stream);
  * (((ceil(K/64)*64*2*N + 255) & ~255) + 4*N bytes, e.g. above 3261 tokens at K = 2560), or
  * whose few-token partial products may not fit (16 KiB per 128-row tile and K slice it may take, e.g.
  * 151936x896 at up to 32 tokens: 38.9 MB), returns TQHIP_ENOSCRATCH before launching
- * anything; no call is rerouted to another kernel (K slices above 32 tokens run one after the
- * other, with the same bits). Group sizes that are not a
+ * anything; no call is rerouted to another kernel (the K slices of a call that does not take the
+ * few-token kernel run one after the other, with the same bits). Group sizes that are not a
  * multiple of 32 run one matvec per token, with kernels that need no scratch. All calls
  * on one GPU share the array: calls that overlap on one GPU (two streams, or two host
  * threads) race and must be ordered by the caller. */

@@ -15,8 +15,8 @@
 // during the current one's MFMAs.
 //
 // A call on host arrays (matmul_vq2) was one matvec per token, each with its own upload, launch,
-// download and wait: 64 tokens through a layer of 896 / 4864 wide matrices took 8350 us. With this
-// kernel it is one of each per matrix, 580 us, of which the seven products take 110 (5-13 us each:
+// download and wait: 64 tokens through a layer of 896 / 4864 wide matrices took 8.5 ms. With this
+// kernel it is one of each per matrix, 590 us, of which the seven products take 114 (5-13 us each:
 // launch and load latency; the matrix instructions alone need 3 us at 4864x896) and the copies
 // the rest.
 

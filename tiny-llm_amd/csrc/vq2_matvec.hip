@@ -899,7 +899,9 @@ __global__ __launch_bounds__(64 * kTabWaves) void vq2_matvec_table(const uint8_t
 // sub-table, 16 or 8 waves) was slower: 35-42 us at 151936x2560.
 constexpr int kSlabDwords = 32;     // index dwords of a slab
 constexpr int kSlabMaxDim = 1 << 20;
-constexpr int kSlabMaxBatches = 3;  // batches per wave (128 VGPRs): <= 768 rows per workgroup
+// Batches per wave: <= 768 rows per workgroup. 16 waves leave 128 VGPRs a lane, past which three batches go by
+// 4 (spilled ahead of the slabs and reloaded once in each); one and two spill nothing.
+constexpr int kSlabMaxBatches = 3;
 
 template <int BMAX>
 __global__ __launch_bounds__(64 * kTabWaves) void vq2_matvec_slabs(const uint8_t *__restrict__ w,
