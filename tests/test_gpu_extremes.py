@@ -96,6 +96,20 @@ def test_non_finite_activation(gpu, orc, name, M, K, off, kind):
     assert bad == 0, f"{name} {kind}: {bad} of {M} outputs finite where the oracle's are not"
 
 
+# groups of 32 and 128: the set kernel (rows of 1, 3 and 5 slots, one that ends inside a group), and with x
+# off 16 bytes the wave-per-row kernel (32) and the split-K and register-path ones (128)
+@pytest.mark.parametrize("g", [32, 128])
+@pytest.mark.parametrize("M,K,off", [(4864, 896, 0), (896, 4864, 0), (2560, 9728, 0), (300, 1000, 0), (896, 896, 1),
+                                     (2560, 9728, 1)])
+def test_wide_range_by_group_size(gpu, orc, monkeypatch, g, M, K, off):
+    print(f"[extremes] groups of {g} {M}x{K} offset {4 * off}", flush=True)
+    monkeypatch.setitem(globals(), "G", g)
+    w, x = gpu.synth_i4(M, K, g, seed=M + K), gpu.synth_normal(K, seed=K + 3)
+    for v, y in ((w, extreme_x(K, seed=K + 1)), (special_headers(w, M, K, seed=M, G=g), x),
+                 (w, (x * np.float32(1e-35)).astype(np.float32))):
+        check(run(gpu, v, y, M, K, off), orc.matvec_i4(v, y, M, K, g, threads=16), f"groups of {g}")
+
+
 @pytest.mark.parametrize("M,K", [(3072, 1024), (32768, 896), (151936, 896), (2001, 3052)])
 @pytest.mark.parametrize("kind", ["nan", "inf"])
 def test_vq2_non_finite_activation(gpu, orc, M, K, kind):

@@ -28,7 +28,8 @@ struct SkinnyGeom {
 // workgroup reads its KS partials of 16 KB alone, 0.33 us each, a step of a slice takes 0.28 us
 // (fitted on MI355X to 896x4864 with 70 / 37 / 22 / 11 slices: 30.0, 19.5, 14.6, 11.7 us). Filling the
 // chip instead, us -> this rule, 8 tokens: 896x896 10.1 -> 7.7, 4864x896 12.0 -> 8.3, 896x4864
-// 30.2 -> 11.7, 2560x4096 19.6 -> 12.0, 2048x2048 17.9 -> 9.4; 9728x2560 and 151936x896 the same.
+// 30.2 -> 11.7, 2560x4096 19.6 -> 12.0, 2048x2048 17.9 -> 9.4; 9728x2560 and 151936x896 the same. Over 14 shapes
+// from 128x896 to 18944x3584 at 2, 8 and 32 tokens one is slower, 2560x9728 at 32: 23.4 -> 23.7.
 inline SkinnyGeom skinny_geom(int M, int K, int cus) {
     SkinnyGeom g;
     g.tiles = (M + kSkRows - 1) / kSkRows;
